@@ -13,6 +13,7 @@
 
 #include "../../include/cunibs_amd.h"
 #include "coil.hpp"
+#include "dipole.hpp"
 #include "prims.hpp"
 #include "recovery.hpp"
 #include "mlp.hpp"
@@ -93,10 +94,10 @@ struct cn_context {
     std::int64_t n_region = 0;
     double region_volume = 0.0;
     // per-block scratch (grow-only)
-    cn::DeviceBuffer<double> d_centers, d_handles, d_dists, d_tf, d_origins;
+    cn::DeviceBuffer<double> d_centers, d_handles, d_dists, d_tf;
     cn::DeviceBuffer<std::int32_t> d_degen;
-    cn::DeviceBuffer<float> d_dip, d_dadt_nodes, d_dadt_elm, d_q, d_B, d_E, d_magn, d_rhs, d_stage;
-    cn::DeviceBuffer<double> d_X, d_v, d_x0;
+    cn::DeviceBuffer<float> d_dadt_nodes, d_dadt_elm, d_q, d_B, d_E, d_magn, d_rhs, d_stage;
+    cn::DeviceBuffer<double> d_X, d_v, d_x0, d_rhs_sums;
     // Sliced ELL copies of the finest level's operator (with its diagonal, for the V-cycle) and of
     // the differenced off-diagonal operator (the block iteration's SpMM); width 0 when not built.
     cn::DeviceBuffer<int2> ell_full, ell_off;
@@ -116,9 +117,12 @@ struct cn_context {
         }
         solver->set_off_ell(max_k > 0 && ell_off_w > 0 ? ell_off.get() : nullptr, ell_off_w, max_k);
     }
-    // Pinned sources of the host-to-device copies a block issues without waiting on them: the
-    // packed dipoles (coil stage, either stream) and the block's own small tables.
-    cn::PinnedStage stage_coil, stage_blk;
+    // The nodes' boxes and the current call's coil, for the N-body (dipole.hip).
+    cn::BoxTree boxes;
+    cn::DipoleSet dipoles;
+    // Pinned source of the host-to-device copies a block issues without waiting on them: its own
+    // small tables.
+    cn::PinnedStage stage_blk;
     // Pipelined sweeps (cn_solve_sweep): the coil stages (dA/dt, element pass, RHS) of the next
     // two blocks run on s2 into their own buffer sets while the current block solves, recovers its
     // field and reduces its metrics on s.
@@ -356,7 +360,8 @@ void build_context(cn_context& c, const double* nodes_mm, std::int64_t n, const 
     tets_in.release();
     tags_in.release();
 
-    lap();  // 2: Morton order
+    build_box_tree(c.boxes, c.nodes.get(), n, s);
+    lap();  // 2: Morton order, boxes
     DeviceBuffer<double> g64(12 * m, "g64"), vols64(m, "vols64"), cond(m, "cond");
     p1_gradients(c.nodes.get(), c.tets.get(), m, g64.get(), vols64.get(), s);
     const int bad = count_bad_volumes(vols64.get(), m, s);
@@ -477,137 +482,6 @@ void build_context(cn_context& c, const double* nodes_mm, std::int64_t n, const 
     d2h(&c.region_volume, vol.get(), 1, s);
     sync(s, "context build");
     lap();  // 8: skin surface, region slice
-}
-
-// Dipoles of one placement in its coil frame, FP64 as fem/placement.py:294-313, then FP32 pack
-// [s | m | m x s | |s|^2] centred at the coil origin.
-// The direction every dipole moment lies along, if there is one (coil models of planar windings
-// put all their moments on the coil normal): |m_j x d| <= 1e-12 |m_j| for all j. Writes the unit
-// direction of the largest moment.
-bool common_moment_direction(const double* mom, std::int64_t n_dip, double* d) {
-    std::int64_t big = 0;
-    double best = 0.0;
-    for (std::int64_t j = 0; j < n_dip; ++j) {
-        const double q = mom[3 * j] * mom[3 * j] + mom[3 * j + 1] * mom[3 * j + 1] + mom[3 * j + 2] * mom[3 * j + 2];
-        if (q > best) {
-            best = q;
-            big = j;
-        }
-    }
-    if (!(best > 0.0)) return false;
-    const double nb = std::sqrt(best);
-    for (int r = 0; r < 3; ++r) d[r] = mom[3 * big + r] / nb;
-    for (std::int64_t j = 0; j < n_dip; ++j) {
-        const double* m = mom + 3 * j;
-        const double cx = m[1] * d[2] - m[2] * d[1], cy = m[2] * d[0] - m[0] * d[2], cz = m[0] * d[1] - m[1] * d[0];
-        const double mm = m[0] * m[0] + m[1] * m[1] + m[2] * m[2];
-        if (cx * cx + cy * cy + cz * cz > 1e-24 * mm) return false;
-    }
-    return true;
-}
-
-// Per placement, for the parallel-moment N-body: -2 s (3), |s|^2, mu, mu s (3) in FP32 with s
-// relative to the coil origin (as pack_dipoles), and the rotated direction.
-void pack_dipoles_parallel(const double* tf, const double* pos_m, const double* mom, std::int64_t n_dip,
-                           const double* dir, float* out, double* origin, float* dir_out) {
-    double rot[3][3], trans[3];
-    for (int r = 0; r < 3; ++r) {
-        for (int q = 0; q < 3; ++q) rot[r][q] = tf[4 * r + q];
-        trans[r] = tf[4 * r + 3];
-    }
-    const double o[3] = {trans[0] * 1e-3, trans[1] * 1e-3, trans[2] * 1e-3};
-    for (int r = 0; r < 3; ++r) origin[r] = o[r];
-    for (int r = 0; r < 3; ++r) {
-        double acc = 0.0;
-        for (int q = 0; q < 3; ++q) acc += dir[q] * rot[r][q];
-        dir_out[r] = static_cast<float>(acc);
-    }
-    for (std::int64_t j = 0; j < n_dip; ++j) {
-        double sd[3];
-        for (int r = 0; r < 3; ++r) {
-            double acc = 0.0;
-            for (int q = 0; q < 3; ++q) acc += pos_m[3 * j + q] * 1e3 * rot[r][q];
-            sd[r] = (acc + trans[r]) * 1e-3 - o[r];
-        }
-        const double mu = mom[3 * j] * dir[0] + mom[3 * j + 1] * dir[1] + mom[3 * j + 2] * dir[2];
-        float* p = out + 8 * j;
-        const float sf[3] = {static_cast<float>(sd[0]), static_cast<float>(sd[1]), static_cast<float>(sd[2])};
-        for (int r = 0; r < 3; ++r) {
-            p[r] = -2.0f * sf[r];
-            p[5 + r] = static_cast<float>(mu * sd[r]);
-        }
-        p[3] = sf[0] * sf[0] + sf[1] * sf[1] + sf[2] * sf[2];
-        p[4] = static_cast<float>(mu);
-    }
-}
-
-// dA/dt at the nodes for k placements (frames tf, k x 16) into out (n, 3, K): the parallel-moment
-// kernel when the coil allows it, the general one otherwise.
-void dadt_for_frames(cn_context& c, const double* tf, int k, int K, const double* pos_m, const double* mom,
-                     std::int64_t n_dip, float scale, float* out, hipStream_t s, int max_blocks = 0);
-
-void pack_dipoles(const double* tf, const double* pos_m, const double* mom, std::int64_t n_dip, float* out,
-                  double* origin) {
-    double rot[3][3], trans[3];
-    for (int r = 0; r < 3; ++r) {
-        for (int q = 0; q < 3; ++q) rot[r][q] = tf[4 * r + q];
-        trans[r] = tf[4 * r + 3];
-    }
-    const double o[3] = {trans[0] * 1e-3, trans[1] * 1e-3, trans[2] * 1e-3};
-    for (int r = 0; r < 3; ++r) origin[r] = o[r];
-    for (std::int64_t j = 0; j < n_dip; ++j) {
-        double s[3], mm[3];
-        for (int r = 0; r < 3; ++r) {
-            double acc = 0.0, am = 0.0;
-            for (int q = 0; q < 3; ++q) {
-                acc += pos_m[3 * j + q] * 1e3 * rot[r][q];
-                am += mom[3 * j + q] * rot[r][q];
-            }
-            s[r] = (acc + trans[r]) * 1e-3 - o[r];
-            mm[r] = am;
-        }
-        const double mxs[3] = {mm[1] * s[2] - mm[2] * s[1], mm[2] * s[0] - mm[0] * s[2], mm[0] * s[1] - mm[1] * s[0]};
-        float* p = out + 10 * j;
-        for (int r = 0; r < 3; ++r) {
-            p[r] = static_cast<float>(s[r]);
-            p[3 + r] = static_cast<float>(mm[r]);
-            p[6 + r] = static_cast<float>(mxs[r]);
-        }
-        p[9] = p[0] * p[0] + p[1] * p[1] + p[2] * p[2];  // from the FP32 positions, as the reference
-    }
-}
-
-void dadt_for_frames(cn_context& c, const double* tf, int k, int K, const double* pos_m, const double* mom,
-                     std::int64_t n_dip, float scale, float* out, hipStream_t s, int max_blocks) {
-    using namespace cn;
-    // The packed dipoles (and the moment directions) and the origins are built in the pinned
-    // stage and copied from there: this function returns before the copies have run.
-    double dir[3];
-    const bool parallel = common_moment_direction(mom, n_dip, dir);
-    const std::size_t n_pack = static_cast<std::size_t>((parallel ? 8 : 10) * n_dip * k);
-    const std::size_t n_dirs = parallel ? 3 * static_cast<std::size_t>(k) : 0;
-    const std::size_t f_bytes = (n_pack + n_dirs) * sizeof(float);
-    const std::size_t o_off = (f_bytes + 15) / 16 * 16;
-    char* host = static_cast<char*>(c.stage_coil.fill(o_off + 3 * sizeof(double) * k));
-    float* dip = reinterpret_cast<float*>(host);
-    double* origins = reinterpret_cast<double*>(host + o_off);
-    for (int i = 0; i < k; ++i) {
-        if (parallel)
-            pack_dipoles_parallel(tf + 16 * i, pos_m, mom, n_dip, dir, dip + 8 * n_dip * i, origins + 3 * i,
-                                  dip + n_pack + 3 * i);
-        else
-            pack_dipoles(tf + 16 * i, pos_m, mom, n_dip, dip + 10 * n_dip * i, origins + 3 * i);
-    }
-    c.d_dip.ensure(n_pack + n_dirs, "dipoles");
-    c.d_origins.ensure(3 * k, "origins");
-    c.stage_coil.send(c.d_dip.get(), 0, f_bytes, s);
-    c.stage_coil.send(c.d_origins.get(), o_off, 3 * sizeof(double) * k, s);
-    c.stage_coil.done(s);
-    if (parallel)
-        dadt_nbody_parallel(c.d_dip.get(), static_cast<int>(n_dip), c.nodes.get(), c.n, c.d_origins.get(),
-                            c.d_dip.get() + n_pack, k, K, scale, out, s, max_blocks);
-    else
-        dadt_nbody(c.d_dip.get(), static_cast<int>(n_dip), c.nodes.get(), c.n, c.d_origins.get(), k, K, scale, out, s);
 }
 
 void place_block(cn_context& c, const double* centers, const double* handles, const double* dists, int k,
@@ -813,24 +687,17 @@ void uq_prepare(cn_context& c, const double* pos_m, const double* mom, std::int6
     place_block(c, center, handle, &dist, 1, tf.data(), degen.data());
     require(handle == nullptr || degen[0] == 0, "degenerate coil placement (handle along the scalp normal)");
     std::copy(tf.begin(), tf.end(), u.transform);
-    std::vector<float> dip(static_cast<std::size_t>(10 * n_dip));
-    std::vector<double> origin(3);
-    pack_dipoles(tf.data(), pos_m, mom, n_dip, dip.data(), origin.data());
-    DeviceBuffer<float> ddip(dip.size(), "dipoles");
-    DeviceBuffer<double> dorg(3, "origin");
-    h2d(ddip.get(), dip.data(), dip.size(), s);
-    h2d(dorg.get(), origin.data(), 3, s);
-    sync(s, "dipole upload");  // the sources are function-local
     u.dadt_nodes1.reset(3 * n, "uq dadt nodes");
-    dadt_nbody(ddip.get(), static_cast<int>(n_dip), c.nodes.get(), n, dorg.get(), 1, 1,
-               static_cast<float>(didt) * static_cast<float>(kMu0Over4Pi), u.dadt_nodes1.get(), s);
+    set_coil(c.dipoles, c.boxes, pos_m, mom, n_dip, s);
+    dadt_block(c.dipoles, c.boxes, c.nodes.get(), n, tf.data(), 1, 1,
+               static_cast<float>(didt) * static_cast<float>(kMu0Over4Pi), u.dadt_nodes1.get(), 0, false, s);
     DeviceBuffer<float> negvc(m, "tissue neg_vc"), q(4 * m, "corner terms");
     for (int t = 0; t < T; ++t) {
         tissue_neg_vc(c.vols32.get(), c.tags.get(), m, present[t], negvc.get(), s);
         element_pass(u.dadt_nodes1.get(), c.tets.get(), c.g32.get(), negvc.get(), m, 1, 1, nullptr, q.get(),
                      c.corner_pos.get(), s);
         node_rhs(q.get(), c.n2c_ptr.get(), n, 1, 1, c.ground, u.rhs.get() + static_cast<std::int64_t>(t) * nr, nullptr,
-                 s);
+                 c.d_rhs_sums, s);
     }
     u.sum.reset(m, "|E| sum");
     u.sumsq.reset(m, "|E| sum of squares");
@@ -1115,7 +982,8 @@ void solve_block(cn_context& c, const double* pos_m, const double* mom, std::int
     c.d_B.ensure(nr * K, "rhs block");
     const float scale = static_cast<float>(didt) * static_cast<float>(kMu0Over4Pi);
     c.mark_phase(1, s);
-    dadt_for_frames(c, tf.data(), k, K, pos_m, mom, n_dip, scale, c.d_dadt_nodes.get(), s);
+    set_coil(c.dipoles, c.boxes, pos_m, mom, n_dip, s);
+    dadt_block(c.dipoles, c.boxes, c.nodes.get(), n, tf.data(), k, K, scale, c.d_dadt_nodes.get(), 0, false, s);
     c.mark_phase(2, s);
     // Per-placement conductivities: the tissue decomposition of the operator and a (K, n_sigma)
     // table for the RHS; padded columns take the context's table.
@@ -1171,7 +1039,7 @@ void solve_block(cn_context& c, const double* pos_m, const double* mom, std::int
         c.d_rhs.ensure(n * k, "rhs full");
         rhs_full = c.d_rhs.get();
     }
-    node_rhs(c.d_q.get(), c.n2c_ptr.get(), n, k, K, c.ground, c.d_B.get(), rhs_full, s);
+    node_rhs(c.d_q.get(), c.n2c_ptr.get(), n, k, K, c.ground, c.d_B.get(), rhs_full, c.d_rhs_sums, s);
     c.mark_phase(3, s);
     // 3. block PCG.
     SolveOptions opt;
@@ -1344,7 +1212,6 @@ void solve_sweep(cn_context& c, const double* pos_m, const double* mom, std::int
                                       ": handle_mm lies on the outward normal through the scalp projection of "
                                       "center_mm, so the coil's rotation about the normal is undefined.");
     if (transforms_out) std::memcpy(transforms_out, tf.data(), sizeof(double) * tf.size());
-    if (c.s2 == nullptr) check(hipStreamCreateWithFlags(&c.s2, hipStreamNonBlocking), "create stream");
     for (auto& e : c.coil_done)
         if (e == nullptr) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "coil event");
     c.d_dadt_nodes.ensure(3 * n * K, "dadt nodes");
@@ -1366,11 +1233,11 @@ void solve_sweep(cn_context& c, const double* pos_m, const double* mom, std::int
     auto coil_stage = [&](int b) {
         const int first = b * block_k, k = std::min(block_k, n_place - first), buf = b % 3;
         const int Kb = padded_width(k);
-        dadt_for_frames(c, tf.data() + 16 * static_cast<std::size_t>(first), k, Kb, pos_m, mom, n_dip, scale,
-                        nodal[buf], c.s2, b == 0 ? 0 : c.coil_blocks);
+        dadt_block(c.dipoles, c.boxes, c.nodes.get(), n, tf.data() + 16 * static_cast<std::size_t>(first), k, Kb, scale,
+                   nodal[buf], b == 0 ? 0 : c.coil_blocks, b > 0, c.s2);
         element_pass(nodal[buf], c.tets.get(), c.g32.get(), c.neg_vc.get(), m, k, Kb, nullptr, c.d_q.get(),
                      c.corner_pos.get(), c.s2);
-        node_rhs(c.d_q.get(), c.n2c_ptr.get(), n, k, Kb, c.ground, rhs[buf], nullptr, c.s2);
+        node_rhs(c.d_q.get(), c.n2c_ptr.get(), n, k, Kb, c.ground, rhs[buf], nullptr, c.d_rhs_sums, c.s2);
         check(hipEventRecord(c.coil_done[buf], c.s2), "coil event");
     };
     SolveOptions opt;
@@ -1399,7 +1266,6 @@ void solve_sweep(cn_context& c, const double* pos_m, const double* mom, std::int
     c.d_magn.ensure(m * K, "magnE");
     if (rec != nullptr) c.d_slots.ensure(3 * rec->n_slots * K, "recovered slots");
     if (rec != nullptr && rec->mode != kRecoveryHarmonic) c.d_Eraw.ensure(3 * m * K, "raw E");
-    if (c.s3 == nullptr) check(hipStreamCreateWithFlags(&c.s3, hipStreamNonBlocking), "create stream");
     for (auto& e : c.solve_done)
         if (e == nullptr) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "solve event");
     const hipStream_t s = c.s, s3 = c.s3;
@@ -1435,6 +1301,7 @@ void solve_sweep(cn_context& c, const double* pos_m, const double* mom, std::int
         // Two coil stages ahead. Block b + 2's is queued after block b has solved and block b - 1's
         // outputs are done, which frees its buffer set; block b's solve writes the solution buffer
         // block b - 2's outputs read, done by then too.
+        set_coil(c.dipoles, c.boxes, pos_m, mom, n_dip, c.s2);
         coil_stage(0);
         if (n_blocks > 1) coil_stage(1);
         for (int b = 0; b < n_blocks; ++b) {
@@ -1543,7 +1410,11 @@ int32_t cn_context_create(const double* nodes_mm, int64_t n_nodes, const int32_t
             cn_default_options(&c->opts);
         cn::require(c->opts.degree >= 1 && c->opts.degree <= cn::kMaxDegree, "degree must be in [1, 6]");
         cn::require(c->opts.lower_ratio > 1.0f, "lower_ratio must exceed 1");
-        cn::check(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking), "create stream");
+        // Together, so that they take different hardware queues (streams are dealt round the queues as
+        // they are created): with several contexts alive, streams created at a sweep's start could share
+        // the queue of the stream they are to run beside.
+        for (hipStream_t* st : {&c->s, &c->s2, &c->s3})
+            cn::check(hipStreamCreateWithFlags(st, hipStreamNonBlocking), "create stream");
         build_context(*c, nodes_mm, n_nodes, tet_nodes, tet_tags, n_tets, skin_tris, n_skin);
         *out = c.release();
     });
@@ -1986,11 +1857,12 @@ int32_t cn_bench_stages(cn_context* c, const double* dip_pos_m, const double* di
         if (rec) c->d_slots.ensure(3 * rec->n_slots * K, "recovered slots");
         if (rec && rec->mode != kRecoveryHarmonic) c->d_Eraw.ensure(3 * m * K, "raw E");
         std::vector<double> met(static_cast<std::size_t>(kMetricsLen) * k);
+        set_coil(c->dipoles, c->boxes, dip_pos_m, dip_moment, n_dip, s);
         auto coil = [&] {
-            dadt_for_frames(*c, frames.data(), k, K, dip_pos_m, dip_moment, n_dip, 0.1f, c->d_dadt_nodes.get(), s);
+            dadt_block(c->dipoles, c->boxes, c->nodes.get(), n, frames.data(), k, K, 0.1f, c->d_dadt_nodes.get(), 0, false, s);
             element_pass(c->d_dadt_nodes.get(), c->tets.get(), c->g32.get(), c->neg_vc.get(), m, k, K, nullptr,
                          c->d_q.get(), c->corner_pos.get(), s, c->vols32.get(), c->tags.get(), nullptr, 0);
-            node_rhs(c->d_q.get(), c->n2c_ptr.get(), n, k, K, c->ground, c->d_B.get(), nullptr, s);
+            node_rhs(c->d_q.get(), c->n2c_ptr.get(), n, k, K, c->ground, c->d_B.get(), nullptr, c->d_rhs_sums, s);
         };
         auto field = [&] {
             if (rec == nullptr)
@@ -2097,8 +1969,9 @@ int32_t cn_bench_dadt(cn_context* c, const double* dip_pos_m, const double* dip_
         for (int i = 0; i < k; ++i) std::copy(tf.begin(), tf.end(), frames.begin() + 16 * i);
         const int K = cn::padded_width(k);
         cn::DeviceBuffer<float> out(3 * c->n * K, "dadt");
+        cn::set_coil(c->dipoles, c->boxes, dip_pos_m, dip_moment, n_dip, s);
         auto run = [&] {
-            dadt_for_frames(*c, frames.data(), k, K, dip_pos_m, dip_moment, n_dip, 1e-7f, out.get(), s);
+            cn::dadt_block(c->dipoles, c->boxes, c->nodes.get(), c->n, frames.data(), k, K, 1e-7f, out.get(), 0, false, s);
         };
         run();
         hipEvent_t e0, e1;

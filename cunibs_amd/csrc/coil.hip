@@ -169,18 +169,12 @@ constexpr int kDadtBlock = 256;
 constexpr int kDipTile = 256;
 constexpr int kNodesPerThread = 8;
 
-// dadt.cu:27-104 restated for CDNA: dipole tiles staged in LDS, 8 nodes per thread in registers,
-// one placement per blockIdx.y. w_j = |r - s_j|^-3 from rn + sn - 2 r.s, FP32, on the vector ALUs.
-// The reciprocal square root is the bare v_rsq_f32 (rsq_normal): rsqrtf wraps the same instruction
-// in a denormal rescale (compare, two multiplies, two selects per pair), and a squared coil-to-node
-// distance is never denormal, so the results are the same bits with a third fewer vector
-// instructions per pair. (Matrix-core versions, with the distances as 16x16x4 FP32 MFMAs and the
-// sums either as MFMAs or on the vector ALUs, measured 0.82-1.35 ms per placement at 1.0M nodes x
-// 2400 dipoles against 0.78 ms for this kernel with rsqrtf, and were dropped.)
-// Output (n, 3, K): the K placements of a node component are contiguous.
-
-// v_rsq_f32 without the denormal rescale; for normal positive inputs it equals rsqrtf bit for bit.
+// The direct sum over dipoles given with their m x s and |s|^2 (dadt.cu:27-104), for the kernel-level
+// entry point; a block's dA/dt is formed in dipole.hip. Dipole tiles staged in LDS, 8 nodes per
+// thread in registers. The reciprocal square root is the bare v_rsq_f32: rsqrtf wraps the same
+// instruction in a denormal rescale, and a squared coil-to-node distance is never denormal.
 __device__ __forceinline__ float rsq_normal(float x) { return __builtin_amdgcn_rsqf(x); }
+
 __global__ void __launch_bounds__(kDadtBlock) dadt_kernel(const float* __restrict__ dip, int n_dip,
                                                           const double* __restrict__ nodes_mm, std::int64_t n,
                                                           const double* __restrict__ origin, float scale, int K,
@@ -252,81 +246,6 @@ __global__ void __launch_bounds__(kDadtBlock) dadt_kernel(const float* __restric
     }
 }
 
-// The same sum when every dipole moment lies along one direction d (planar windings: the moments
-// are the coil normal scaled by mu_j). Then W = d S0 and P = d x S with S0 = sum_j w_j mu_j and
-// S = sum_j w_j mu_j s_j, so dA/dt = scale d x (S0 r - S): four multiply-adds per pair instead of
-// six. Per dipole (FP32): -2 s (3), |s|^2, mu, mu s (3); d per placement. The distance keeps the
-// reference's rn + sn - 2 r.s form.
-__global__ void __launch_bounds__(kDadtBlock) dadt_parallel_kernel(const float* __restrict__ dip, int n_dip,
-                                                                   const double* __restrict__ nodes_mm, std::int64_t n,
-                                                                   const double* __restrict__ origin,
-                                                                   const float* __restrict__ dirs, float scale, int K,
-                                                                   float* __restrict__ out) {
-    __shared__ float4 s_a[kDipTile];  // -2 sx, -2 sy, -2 sz, |s|^2
-    __shared__ float4 s_m[kDipTile];  // mu, mu sx, mu sy, mu sz
-    const int c = blockIdx.y;
-    const float* dp = dip + static_cast<std::int64_t>(c) * n_dip * 8;
-    const double ox = origin[3 * c], oy = origin[3 * c + 1], oz = origin[3 * c + 2];
-    // A thread's nodes are t, t + NT, t + 2 NT, ...; a grid smaller than NT threads walks the
-    // slots in block-uniform steps (so every thread meets the same barriers).
-    const std::int64_t NT = (n + kNodesPerThread - 1) / kNodesPerThread;
-    const float dx = dirs[3 * c], dy = dirs[3 * c + 1], dz = dirs[3 * c + 2];
-    for (std::int64_t slot0 = static_cast<std::int64_t>(blockIdx.x) * blockDim.x; slot0 < NT;
-         slot0 += static_cast<std::int64_t>(gridDim.x) * blockDim.x) {
-        const std::int64_t t = slot0 + threadIdx.x;
-        const std::int64_t T = NT;
-        float rx[kNodesPerThread], ry[kNodesPerThread], rz[kNodesPerThread], rn[kNodesPerThread];
-        float s0[kNodesPerThread], sx[kNodesPerThread], sy[kNodesPerThread], sz[kNodesPerThread];
-#pragma unroll
-        for (int k = 0; k < kNodesPerThread; ++k) {
-            const std::int64_t node = t + k * T;
-            rx[k] = ry[k] = rz[k] = rn[k] = 0.f;
-            if (node < n) {
-                rx[k] = static_cast<float>(nodes_mm[3 * node] * 1e-3 - ox);
-                ry[k] = static_cast<float>(nodes_mm[3 * node + 1] * 1e-3 - oy);
-                rz[k] = static_cast<float>(nodes_mm[3 * node + 2] * 1e-3 - oz);
-                rn[k] = fmaf(rz[k], rz[k], fmaf(ry[k], ry[k], rx[k] * rx[k]));
-            }
-            s0[k] = sx[k] = sy[k] = sz[k] = 0.f;
-        }
-        for (int base = 0; base < n_dip; base += kDipTile) {
-            const int tile = min(kDipTile, n_dip - base);
-            __syncthreads();
-            for (int i = threadIdx.x; i < tile; i += kDadtBlock) {
-                const float* d = dp + static_cast<std::int64_t>(base + i) * 8;
-                s_a[i] = make_float4(d[0], d[1], d[2], d[3]);
-                s_m[i] = make_float4(d[4], d[5], d[6], d[7]);
-            }
-            __syncthreads();
-#pragma unroll 4
-            for (int j = 0; j < tile; ++j) {
-                const float4 a = s_a[j], m = s_m[j];
-#pragma unroll
-                for (int k = 0; k < kNodesPerThread; ++k) {
-                    const float q = fmaf(rz[k], a.z, fmaf(ry[k], a.y, fmaf(rx[k], a.x, a.w)));
-                    const float inv = rsq_normal(q + rn[k]);
-                    const float w = inv * inv * inv;
-                    s0[k] = fmaf(w, m.x, s0[k]);
-                    sx[k] = fmaf(w, m.y, sx[k]);
-                    sy[k] = fmaf(w, m.z, sy[k]);
-                    sz[k] = fmaf(w, m.w, sz[k]);
-                }
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < kNodesPerThread; ++k) {
-            const std::int64_t node = t + k * T;
-            if (node < n) {
-                const float fx = s0[k] * rx[k] - sx[k], fy = s0[k] * ry[k] - sy[k], fz = s0[k] * rz[k] - sz[k];
-                float* o = out + node * 3 * K + c;
-                o[0] = scale * (dy * fz - dz * fy);
-                o[K] = scale * (dz * fx - dx * fz);
-                o[2 * K] = scale * (dx * fy - dy * fx);
-            }
-        }
-    }
-}
-
 // Element pass over (element, placement), placements fastest so the K lanes of an element read
 // and write contiguous memory:
 //   dadt_elm = mean of the four nodal vectors       (dadt_element.cu:6-21)
@@ -366,17 +285,76 @@ __global__ void element_pass_kernel(const float* __restrict__ nodal, const std::
 
 // Node gather (rhs.cu:84-104): b[node] = sum of its corners' q in node2corner order, written to
 // the solver block with the ground row dropped, and optionally to (k, n) full-node storage. The
-// element pass stored the corner terms in that order, so a node's terms are one contiguous run.
+// element pass stored the corner terms in that order, so a node's terms are one contiguous run. A
+// block takes kRhsRows nodes and writes their columns' FP64 sums (fixed tree) to sums (blocks, K).
+constexpr int kRhsRows = kWave;
+
 __global__ void node_rhs_kernel(const float* __restrict__ q, const std::int32_t* __restrict__ ptr, std::int64_t n,
-                                int k, int K, int ground, float* __restrict__ B, float* __restrict__ b_full) {
-    const std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n * K) return;
-    const std::int64_t node = t / K;
-    const int c = static_cast<int>(t % K);
-    float acc = 0.f;
-    for (int p = ptr[node]; p < ptr[node + 1]; ++p) acc += q[static_cast<std::int64_t>(p) * K + c];
-    if (b_full != nullptr && c < k) b_full[c * n + node] = acc;
-    if (node != ground) B[(node - (node > ground)) * K + c] = acc;
+                                int k, int K, int ground, float* __restrict__ B, float* __restrict__ b_full,
+                                double* __restrict__ sums) {
+    __shared__ float tile[32][kRhsRows + 1];  // K <= 32
+    const std::int64_t n0 = static_cast<std::int64_t>(blockIdx.x) * kRhsRows;
+    for (int t = threadIdx.x; t < kRhsRows * K; t += blockDim.x) {
+        const std::int64_t node = n0 + t / K;
+        const int c = t % K;
+        float acc = 0.f;
+        if (node < n) {
+            for (int p = ptr[node]; p < ptr[node + 1]; ++p) acc += q[static_cast<std::int64_t>(p) * K + c];
+            if (b_full != nullptr && c < k) b_full[c * n + node] = acc;
+            if (node != ground) B[(node - (node > ground)) * K + c] = acc;
+        }
+        tile[c][t / K] = acc;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1), waves = blockDim.x / kWave;
+    for (int c = threadIdx.x / kWave; c < K; c += waves) {
+        double v = static_cast<double>(tile[c][lane]);
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + c] = v;
+    }
+}
+
+// The right-hand side of a field without sources sums to zero over all nodes; its FP32 rounding
+// does not, and whatever is left (5e-8 of the norm) flows to the ground node, which shifts the whole
+// potential by 1e-6 to 4e-5 of its norm. The sum of each column is taken back from kBalanceRows rows
+// spread over the mesh, each rounded value's error carried to the next, which leaves less than one
+// rounding of one entry (the potential's error: 3e-7, that of the solve). One block per column; the
+// sum does not depend on the block's width.
+constexpr int kBalanceRows = kBlock;
+
+__global__ void __launch_bounds__(kBlock) balance_rhs_kernel(const double* __restrict__ sums, std::int64_t blocks,
+                                                             std::int64_t n, int K, int ground, float* __restrict__ B,
+                                                             float* __restrict__ b_full) {
+    __shared__ double s[kBlock];
+    __shared__ float v[kBalanceRows];
+    const int c = blockIdx.x, t = threadIdx.x;
+    double acc = 0.0;
+    for (std::int64_t b = t; b < blocks; b += kBlock) acc += sums[b * K + c];
+    s[t] = acc;
+    const std::int64_t nr = n - 1;
+    const int rows = static_cast<int>(min(static_cast<std::int64_t>(kBalanceRows), nr));
+    const std::int64_t row = static_cast<std::int64_t>(t) * nr / rows;
+    if (t < rows) v[t] = B[row * K + c];
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if (t < w) s[t] += s[t + w];
+        __syncthreads();
+    }
+    if (t == 0 && s[0] != 0.0) {
+        const double share = -s[0] / rows;
+        double carry = 0.0;
+        for (int i = 0; i < rows; ++i) {
+            const double x = static_cast<double>(v[i]) + (share + carry);
+            v[i] = static_cast<float>(x);
+            carry = x - static_cast<double>(v[i]);
+        }
+    }
+    __syncthreads();
+    if (t < rows) {
+        B[row * K + c] = v[t];
+        if (b_full != nullptr) b_full[c * n + row + (row >= ground)] = v[t];
+    }
 }
 
 __global__ void corner_pos_kernel(const std::int32_t* __restrict__ idx, std::int64_t count,
@@ -409,15 +387,6 @@ void dadt_nbody(const float* dip, int n_dip, const double* nodes_mm, std::int64_
     dadt_kernel<<<dim3(gx, k), kDadtBlock, 0, s>>>(dip, n_dip, nodes_mm, n, origins, scale, K, out);
 }
 
-void dadt_nbody_parallel(const float* dip8, int n_dip, const double* nodes_mm, std::int64_t n, const double* origins,
-                         const float* dirs, int k, int K, float scale, float* out, hipStream_t s, int max_blocks) {
-    if (n <= 0 || k <= 0) return;
-    const std::int64_t threads = (n + kNodesPerThread - 1) / kNodesPerThread;
-    unsigned gx = grid_for(threads, kDadtBlock);
-    if (max_blocks > 0) gx = std::max(1u, std::min(gx, static_cast<unsigned>((max_blocks + k - 1) / k)));
-    dadt_parallel_kernel<<<dim3(gx, k), kDadtBlock, 0, s>>>(dip8, n_dip, nodes_mm, n, origins, dirs, scale, K, out);
-}
-
 void element_pass(const float* nodal, const std::int32_t* tets, const float* g, const float* neg_vc, std::int64_t m,
                   int k, int K, float* elm, float* q, const std::int32_t* corner_pos, hipStream_t s, const float* vols,
                   const std::int32_t* tags, const float* sigma_tag, int n_sigma) {
@@ -431,8 +400,14 @@ void corner_positions(const std::int32_t* idx, std::int64_t count, std::int32_t*
 }
 
 void node_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int k, int K, int ground, float* B,
-              float* b_full, hipStream_t s) {
-    if (const unsigned gr = grid_for(n * K)) node_rhs_kernel<<<gr, kBlock, 0, s>>>(q, ptr, n, k, K, ground, B, b_full);
+              float* b_full, DeviceBuffer<double>& sums, hipStream_t s) {
+    const std::int64_t blocks = (n + kRhsRows - 1) / kRhsRows;
+    if (blocks <= 0) return;
+    sums.ensure(static_cast<std::size_t>(blocks) * K, "right-hand-side sums");
+    node_rhs_kernel<<<static_cast<unsigned>(blocks), std::min(kRhsRows * K, 1024), 0, s>>>(q, ptr, n, k, K, ground, B,
+                                                                                          b_full, sums.get());
+    if (n > 1 && k > 0)
+        balance_rhs_kernel<<<static_cast<unsigned>(k), kBlock, 0, s>>>(sums.get(), blocks, n, K, ground, B, b_full);
 }
 
 }  // namespace cn

@@ -16,12 +16,6 @@ void place_transforms(const double* centers, const double* handles, const double
 // dip: per placement n_dip x [s(3) m(3) m x s(3) |s|^2] FP32, centred at that placement's origin.
 void dadt_nbody(const float* dip, int n_dip, const double* nodes_mm, std::int64_t n, const double* origins, int k,
                 int K, float scale, float* out, hipStream_t s);
-// All moments along one direction per placement (dirs: k x 3): dip8 per placement n_dip x
-// [-2 s(3) |s|^2 mu mu s(3)] FP32.
-// max_blocks > 0 caps the grid (all k placements together) and the blocks walk the nodes: a
-// smaller footprint for running beside other work.
-void dadt_nbody_parallel(const float* dip8, int n_dip, const double* nodes_mm, std::int64_t n, const double* origins,
-                         const float* dirs, int k, int K, float scale, float* out, hipStream_t s, int max_blocks = 0);
 // Element average of the nodal dA/dt and the RHS corner terms; sigma_tag (K x n_sigma FP32, with
 // vols and tags) gives each placement its own conductivities instead of neg_vc. The corner term of
 // corner 4 e + i is stored at row corner_pos[4 e + i] of q: its position in node2corner order.
@@ -31,9 +25,10 @@ void element_pass(const float* nodal, const std::int32_t* tets, const float* g, 
                   int n_sigma = 0);
 // corner_pos[idx[p]] = p for the 4m corners of a node2corner list.
 void corner_positions(const std::int32_t* idx, std::int64_t count, std::int32_t* corner_pos, hipStream_t s);
-// b[node] = sum of the node's corner terms, q in node2corner order (rows ptr[node] .. ptr[node+1]).
+// b[node] = sum of the node's corner terms, q in node2corner order (rows ptr[node] .. ptr[node+1]),
+// each column brought to a zero sum over all nodes; `sums` is scratch (grow-only).
 void node_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int k, int K, int ground, float* B,
-              float* b_full, hipStream_t s);
+              float* b_full, DeviceBuffer<double>& sums, hipStream_t s);
 
 // post.hip
 void scatter_potential(const double* X, std::int64_t n, int k, int K, int ground, double* v, hipStream_t s);

@@ -89,6 +89,7 @@ struct Hierarchy {
 };
 
 // ---------------- mesh.hip ----------------
+void bounding_box(const double* pts, std::int64_t n, double* lo, double* span, hipStream_t s);
 void morton_keys(const double* pts, std::int64_t n, std::uint64_t* keys, hipStream_t s);
 void tet_lowest_node(const std::int32_t* inverse, const std::int32_t* tets, std::int64_t m,
                      std::uint32_t* lowest, hipStream_t s);

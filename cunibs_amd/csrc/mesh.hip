@@ -434,25 +434,31 @@ __global__ void tri_vertices_kernel(const double* __restrict__ nodes, const std:
 // Host launchers
 // ----------------------------------------------------------------------------------------------
 
-void morton_keys(const double* pts, std::int64_t n, std::uint64_t* keys, hipStream_t s) {
-    if (n <= 0) return;
+// Lower corner and extents (at least 1e-12) of the points' bounding box; waits on s.
+void bounding_box(const double* pts, std::int64_t n, double* lo, double* span, hipStream_t s) {
     const int blocks = static_cast<int>(std::min<std::int64_t>(grid_for(n), 1024));
     DeviceBuffer<double> part(6 * static_cast<std::size_t>(blocks), "bbox partials");
     bbox_kernel<<<blocks, kBlock, 0, s>>>(pts, n, part.get());
     std::vector<double> h(6 * static_cast<std::size_t>(blocks));
     d2h(h.data(), part.get(), h.size(), s);
     sync(s, "bbox");
-    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    double hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int a = 0; a < 3; ++a) lo[a] = INFINITY;
     for (int b = 0; b < blocks; ++b)
         for (int a = 0; a < 3; ++a) {
             lo[a] = std::min(lo[a], h[6 * b + a]);
             hi[a] = std::max(hi[a], h[6 * b + 3 + a]);
         }
-    double sp[3];
     for (int a = 0; a < 3; ++a) {
-        sp[a] = hi[a] - lo[a];
-        if (!(sp[a] > 1e-12)) sp[a] = 1e-12;
+        span[a] = hi[a] - lo[a];
+        if (!(span[a] > 1e-12)) span[a] = 1e-12;
     }
+}
+
+void morton_keys(const double* pts, std::int64_t n, std::uint64_t* keys, hipStream_t s) {
+    if (n <= 0) return;
+    double lo[3], sp[3];
+    bounding_box(pts, n, lo, sp, s);
     morton_kernel<<<grid_for(n), kBlock, 0, s>>>(pts, n, lo[0], lo[1], lo[2], sp[0], sp[1], sp[2], keys);
 }
 

@@ -1467,6 +1467,80 @@ __global__ void __launch_bounds__(kWave) round_start_kernel(int k, double tolera
     if (t == 0) state[0] = active_cols == 0;
 }
 
+// The constant part of a solution's error. The ground node takes whatever net current the residual has
+// left, so the whole potential is off by that over the ground's conductance, 4e-6 to 4e-5 of its norm
+// after a solve to 1e-6 where the rest of the error is 5e-7. With 1 the vector of ones,
+// x += 1 (1^T r) / (1^T A 1) takes it out (the A-norm projection of the error on 1; the residual changes
+// in the ground's own neighbours alone, by a twentieth of the tolerance; a column that it would take
+// above the tolerance, as a dipole all but touching a node can, keeps its solution). A is symmetric, so 1^T r is
+// sum_i (b_i - s_i x_i) with the row sums s = A 1, a pass over two vectors. (The recursive residual's sum
+// will not do: its FP32 rounding since the first iteration is what there is to take out.)
+
+// sums[block, c] = sum over the block's kWave rows of b - s x in FP64 (of s alone without b), a fixed
+// tree whatever K. s is (n), or (n, K) with SK.
+template <int K, bool SK>
+__global__ void __launch_bounds__((kWave * K < 1024 ? kWave * K : 1024)) column_sum_kernel(
+    std::int64_t n, const float* __restrict__ b, const float* __restrict__ s, const double* __restrict__ x,
+    double* __restrict__ sums) {
+    __shared__ double tile[K][kWave + 1];
+    const std::int64_t r0 = static_cast<std::int64_t>(blockIdx.x) * kWave;
+    for (int t = threadIdx.x; t < kWave * K; t += blockDim.x) {
+        const std::int64_t row = r0 + t / K, at = row * K + t % K;
+        double v = 0.0;
+        if (row < n) {
+            const double sv = static_cast<double>(s[SK ? at : row]);
+            v = b != nullptr ? fma(-sv, x[at], static_cast<double>(b[at])) : sv;
+        }
+        tile[t % K][t / K] = v;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int c = threadIdx.x / kWave; c < K; c += blockDim.x / kWave) {
+        double v = tile[c][lane];
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + c] = v;
+    }
+}
+
+// out[c] = sum of the block sums of column c (one block per column, fixed order), over den[c * den_step]
+// when den is given (0 where that is not positive).
+__global__ void __launch_bounds__(kBlock) column_total_kernel(const double* __restrict__ sums, std::int64_t blocks,
+                                                              int K, const double* __restrict__ den, int den_step,
+                                                              double* __restrict__ out) {
+    __shared__ double s[kBlock];
+    const int c = blockIdx.x;
+    double acc = 0.0;
+    for (std::int64_t b = threadIdx.x; b < blocks; b += kBlock) acc += sums[b * K + c];
+    s[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    const double d = den != nullptr ? den[c * den_step] : 1.0;
+    out[c] = d > 0.0 ? s[0] / d : 0.0;
+}
+
+// The shifts of the columns whose residual they took above the tolerance, to be undone; 0 elsewhere.
+__global__ void undo_shift_kernel(int K, double tolerance, const double* __restrict__ norms,
+                                  const double* __restrict__ bnorm, double* __restrict__ shift) {
+    const int c = threadIdx.x;
+    if (c < K) shift[c] = norms[c] > tolerance * bnorm[c] ? -shift[c] : 0.0;
+}
+
+// X = out = X + shift per column: the solution handed out, in place of a plain copy.
+template <int K>
+__global__ void shift_copy_kernel(std::int64_t count, const double* __restrict__ shift, double* __restrict__ X,
+                                  double* __restrict__ out) {
+    const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const double v = X[i] + shift[i % K];
+    X[i] = v;
+    out[i] = v;
+}
+
 std::int64_t gram_rows(std::int64_t n) { return (n + kGramBlocks - 1) / kGramBlocks; }
 
 // Sub-lanes per column group (G = K / V groups per row) for a level's row kernels: enough that
@@ -1789,6 +1863,8 @@ void BlockSolver::ensure(int K) {
     norms_.reset(K, "norms");
     bnorm_.reset(K, "right-hand-side norms");
     target_.reset(K, "targets");
+    shift_.reset(2 * static_cast<std::size_t>(K), "solution shifts");
+    col_sums_.reset(static_cast<std::size_t>((n() + kWave - 1) / kWave) * K, "column sums");
     state_.reset(2 + 2 * kMaxBlock, "solver state");
     cap_k_ = K;
     drop_graphs();  // the captured iterations named the buffers just replaced
@@ -2037,6 +2113,7 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
     std::vector<int> host_state(2 + 2 * kMaxBlock, 0);
     bool use_graph = opt.use_graph;  // cleared for the rest of this solve if a capture fails
     int total_iters = 0;
+    bool handed_out = false;  // X holds the solution (written with the round's shift)
     std::vector<int> col_iters(K, 0);
     int slot = 0;
     while (kBlockWidths[slot] != K) ++slot;
@@ -2164,7 +2241,42 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
             sync(s_, "right-hand-side norms");
             check_bnorm();
         }
+        {  // the constant part of the error, and the solution handed out
+            const std::int64_t blocks = (nn + kWave - 1) / kWave;
+            constexpr int kSumThreads = kWave * K < 1024 ? kWave * K : 1024;
+            double* const shift = shift_.get();
+            const double* den = ground_g_.get();
+            const auto sum = [&](auto sk, const float* b, const float* rs) {
+                column_sum_kernel<K, decltype(sk)::value><<<static_cast<unsigned>(blocks), kSumThreads, 0, s_>>>(
+                    nn, b, rs, Xi, col_sums_.get());
+            };
+            if (multi_) {
+                sum(std::true_type{}, nullptr, multi_->rowsum);
+                column_total_kernel<<<K, kBlock, 0, s_>>>(col_sums_.get(), blocks, K, nullptr, 0, shift + K);
+                den = shift + K;
+                sum(std::true_type{}, B, multi_->rowsum);
+            } else {
+                if (!den) {  // once per solver: its operator does not change
+                    ground_g_.reset(1, "ground conductance");
+                    column_sum_kernel<1, false><<<static_cast<unsigned>(blocks), kWave, 0, s_>>>(
+                        nn, nullptr, op_.rowsum, nullptr, col_sums_.get());
+                    column_total_kernel<<<1, kBlock, 0, s_>>>(col_sums_.get(), blocks, 1, nullptr, 0, ground_g_.get());
+                    den = ground_g_.get();
+                }
+                sum(std::false_type{}, B, op_.rowsum);
+            }
+            column_total_kernel<<<K, kBlock, 0, s_>>>(col_sums_.get(), blocks, K, den, multi_ ? 1 : 0, shift);
+            shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift, Xi, X);
+            handed_out = true;
+        }
         true_residual(false);
+        bool over = false;
+        for (int c = 0; c < k; ++c) over |= !(rnorm[c] <= opt.tolerance * bnorm[c]);
+        if (over) {
+            undo_shift_kernel<<<1, kWave, 0, s_>>>(K, opt.tolerance, norms_.get(), bnorm_.get(), shift_.get());
+            shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift_.get(), Xi, X);
+            true_residual(false);
+        }
         double worst = 0.0;
         for (int c = 0; c < k; ++c) worst = std::max(worst, rnorm[c] / bnorm[c]);
         if (stats.refinements < kMaxRounds) {
@@ -2178,8 +2290,10 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
         stats.column_iterations[c] = col_iters[c];
     }
     stats.iterations = total_iters;
-    d2d(X, Xi, static_cast<std::size_t>(nk), s_);
-    sync(s_, "solution copy");
+    if (!handed_out) {
+        d2d(X, Xi, static_cast<std::size_t>(nk), s_);
+        sync(s_, "solution copy");
+    }
     return stats;
 }
 

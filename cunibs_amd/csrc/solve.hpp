@@ -240,6 +240,7 @@ class BlockSolver {
     DeviceBuffer<double> partials_;  // kGramBlocks * 2 * K * K
     DeviceBuffer<double> red_;       // the partials summed over the blocks (2 K^2)
     DeviceBuffer<double> G_, TT_, AL_, D_, norms_, target_;  // AL_: kLag K x K coefficient slots
+    DeviceBuffer<double> shift_, col_sums_, ground_g_;  // the final constant shift of each column
     DeviceBuffer<double> bnorm_;  // ||b_c||, kept on the device for the first round's targets
     DeviceBuffer<float> g_x_[2], g_b_[2];  // the guess basis: FP32 solutions and their right-hand sides
     DeviceBuffer<double> g_mat_;           // its Grams, cross blocks and the last guess's coefficients

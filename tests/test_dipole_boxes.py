@@ -1,0 +1,84 @@
+"""The block N-body (csrc/dipole.hip) against the dipoles' closed form in FP64, with and without the
+box method, at the sizes where its parts change: the widths at which waves share a placement, ragged
+widths, the smallest coil the boxes take, coils whose moments are parallel and not, and the two
+depths of the boxes."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cunibs_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", params=[8.0, 3.2, 2.0])  # below the box method, three levels, four
+def ctx(request):
+    from cunibs_amd import fem
+    head = synthetic.shell_head(request.param, perturb_rms_mm=1.0, seed=2)
+    c = fem.SolverContext(head.nodes_mm, head.tet_nodes, head.tet_tags, head.skin_tris)
+    yield c
+    c.free()
+
+
+def nodal(ctx, pos, mom, sites):
+    from cunibs_amd import fem
+    ex = {"dadt_nodes": 1}
+    res = fem.solve_placements_block(ctx, pos, mom, sites, 1e6, magnitude=False, metrics=False, extra=ex,
+                                     tolerance=0.5)  # the solve itself is not looked at
+    return ex["dadt_nodes"], [r.transform for r in res]
+
+
+def closed_form(pos, mom, tf, nodes_mm):
+    s = pos @ tf[:3, :3].T + tf[:3, 3] * 1e-3
+    m = mom @ tf[:3, :3].T
+    out = np.empty((nodes_mm.shape[0], 3))
+    for i, x in enumerate(nodes_mm * 1e-3):
+        d = x - s
+        out[i] = 0.1 * (np.cross(m, d) / (np.linalg.norm(d, axis=1) ** 3)[:, None]).sum(0)
+    return out
+
+
+@pytest.mark.parametrize("k,dipoles,bent", [(1, 2400, False), (1, 256, True), (2, 255, False), (3, 257, True),
+                                            (5, 600, False), (8, 1002, True), (17, 300, False)])
+def test_block_dadt_matches_the_closed_form(ctx, k, dipoles, bent):
+    coil = synthetic.figure8_coil(seed=3, per_layer=-(-dipoles // 6))
+    pos, mom = coil.positions_m[:dipoles].copy(), coil.moments[:dipoles].copy()
+    if bent:
+        mom += 0.1 * np.abs(mom).max() * np.random.default_rng(1).standard_normal(mom.shape)
+    sites = synthetic.cap_sites(k, seed=k, distance_range_mm=(3.0, 8.0))
+    got, tf = nodal(ctx, pos, mom, sites)
+    rng = np.random.default_rng(0)
+    pick = np.unique(np.concatenate([rng.integers(0, ctx.n_nodes, 600), [0, ctx.n_nodes - 1],
+                                     np.argsort(ctx.nodes_mm[:, 2])[-200:]]))
+    for i in range(k):
+        want = closed_form(pos, mom, tf[i], ctx.nodes_mm[pick])
+        err = np.linalg.norm(got[i][pick] - want, axis=1)
+        # 2-norm: the truncation of the boxes (1e-7 of the field) and FP32 pair terms whose r - s is
+        # rounded to 2^-24 of 0.1 m: 6e-9 m over the 3 mm of the closest pairs, three times in the cube.
+        assert np.linalg.norm(err) <= 6e-6 * np.linalg.norm(want)
+        # At a single node the contributions of the two wings cancel; bounded by the field's scale there.
+        assert err.max() <= 2e-5 * np.abs(want).max()
+
+
+def test_a_placement_does_not_depend_on_its_block(ctx):
+    coil = synthetic.figure8_coil(seed=4)
+    sites = synthetic.cap_sites(9, seed=5)
+    whole, _ = nodal(ctx, coil.positions_m, coil.moments, sites)
+    for lo, hi in ((0, 1), (1, 3), (3, 8)):  # waves share a placement eight, four and two ways
+        part, _ = nodal(ctx, coil.positions_m, coil.moments, sites[lo:hi])
+        np.testing.assert_array_equal(part, whole[lo:hi])
+
+
+@pytest.mark.parametrize("k", [1, 3, 17])
+def test_right_hand_sides_sum_to_zero(ctx, k):
+    """A field without sources puts no net current into the head: what FP32 rounding leaves of the sum
+    is taken back, to one rounding (2^-24) of the largest entry and of the ground node's own."""
+    from cunibs_amd import fem
+    coil = synthetic.figure8_coil(seed=6)
+    ex = {"rhs": 1}
+    fem.solve_placements_block(ctx, coil.positions_m, coil.moments, synthetic.cap_sites(k, seed=k), 1e6,
+                               magnitude=False, metrics=False, extra=ex, tolerance=0.5)
+    b = ex["rhs"].astype(np.float64)
+    assert np.all(np.abs(b.sum(1)) <= 2.0 * 2.0**-24 * np.abs(b).max(1))
