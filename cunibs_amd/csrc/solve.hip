@@ -1922,28 +1922,39 @@ void BlockSolver::set_coarse_sub(int sub) {
     drop_graphs();
 }
 
-template <int K>
-void BlockSolver::build_tail_k(int t) {
+void BlockSolver::build_tail(int t) {
+    // Formed kTailWidth columns a time in vectors of its own, whatever width the solver has allocated:
+    // a level of 1,661 rows takes 52 cycles, 5 ms, where a context of single placements ran one
+    // cycle a column (59 ms). The columns do not depend on the widths solved before.
+    constexpr int K = kTailWidth;
     const int nt = static_cast<int>(h_.levels[t].a.n);
     const int nq = (nt + 3) / 4;
     const std::size_t size = static_cast<std::size_t>((nt + 15) / 16) * nq * kWave;
     std::vector<int> subs(h_.levels.size());
-    for (std::size_t i = 0; i < h_.levels.size(); ++i)
+    std::vector<DeviceBuffer<float>> lb(h_.levels.size()), lx(h_.levels.size()), lr(h_.levels.size());
+    for (std::size_t i = 0; i < h_.levels.size(); ++i) {
         subs[i] = choose_sub(h_.levels[i].a.n, h_.levels[i].a.nnz, col_groups<K>(), n_cu_);
-    if (coarse_sub_ > 0)
-        for (std::size_t i = 1; i < subs.size(); ++i) subs[i] = std::min(coarse_sub_, kWave / col_groups<K>());
+        if (coarse_sub_ > 0 && i > 0) subs[i] = std::min(coarse_sub_, kWave / col_groups<K>());
+        if (static_cast<int>(i) < t) continue;
+        const std::size_t ln = static_cast<std::size_t>(h_.levels[i].a.n) * K;
+        lb[i].reset(ln, "tail level b");
+        lx[i].reset(ln, "tail level x");
+        lr[i].reset(ln, "tail level r");
+    }
+    const std::size_t nc = static_cast<std::size_t>(std::max<std::int64_t>(h_.n_coarse(), 1)) * K;
+    DeviceBuffer<float> cb(nc, "tail coarse b"), cx(nc, "tail coarse x");
     tail_.m.reset(size, "dense tail");
-    check(hipMemsetAsync(tail_.m.get(), 0, sizeof(float) * size, s_), "dense tail clear");
+    zero_f32_kernel<<<grid_for(static_cast<std::int64_t>(size)), kBlock, 0, s_>>>(static_cast<std::int64_t>(size),
+                                                                                 tail_.m.get());
     DeviceBuffer<float> e(static_cast<std::size_t>(nt) * K, "identity block"), xo(static_cast<std::size_t>(nt) * K,
                                                                                    "tail columns");
     const unsigned g = grid_for(static_cast<std::int64_t>(nt) * K);
     for (int c0 = 0; c0 < nt; c0 += K) {
         identity_cols_kernel<K><<<g, kBlock, 0, s_>>>(nt, c0, e.get());
-        run_vcycle<K>(h_, subs, lb_, lx_, lr_, cb_.get(), cx_.get(), e.get(), xo.get(), nullptr, n_cu_, s_, t,
-                      nullptr);
+        run_vcycle<K>(h_, subs, lb, lx, lr, cb.get(), cx.get(), e.get(), xo.get(), nullptr, n_cu_, s_, t, nullptr);
         scatter_cols_kernel<K><<<g, kBlock, 0, s_>>>(nt, nq, c0, xo.get(), tail_.m.get());
     }
-    sync(s_, "dense tail");  // e and xo are freed on return
+    sync(s_, "dense tail");  // the vectors are freed on return
     tail_.level = t;
     tail_.n = nt;
     tail_.nq = nq;
@@ -1953,17 +1964,11 @@ void BlockSolver::ensure_tail() {
     if (tail_ready_) return;
     tail_.level = -1;
     if (tail_on_) {
-        int t = -1;
         for (std::size_t i = 0; i < h_.levels.size(); ++i) {
             if (h_.levels[i].a.n <= kDenseTailMaxRows) {
-                t = static_cast<int>(i);
+                build_tail(static_cast<int>(i));
                 break;
             }
-        }
-        if (t >= 0) {
-            if (cap_k_ < 1) ensure(1);
-            // Formed at the widest allocated width up to 16: the columns of M do not depend on it.
-            dispatch_k(std::min(cap_k_, 16), [&](auto kc) { build_tail_k<decltype(kc)::value>(t); });
         }
     }
     tail_ready_ = true;

@@ -44,6 +44,7 @@ struct DenseTail {
     DeviceBuffer<float> m;
 };
 constexpr int kDenseTailMaxRows = 4096;
+constexpr int kTailWidth = 32;  // columns of the identity taken through the cycle at a time
 
 // The inner margin by block width. A column above the tolerance after a round starts another
 // round, so the margin trades iterations against extra rounds. Up to 16 columns the FP64 true
@@ -211,8 +212,7 @@ class BlockSolver {
     // Form the dense tail if it is on and not current (never during a capture: solve entry points
     // call it before any launch).
     void ensure_tail();
-    template <int K>
-    void build_tail_k(int t);
+    void build_tail(int t);
 
     Operator op_;
     const Hierarchy& h_;
