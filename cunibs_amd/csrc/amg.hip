@@ -477,6 +477,15 @@ __global__ void gather_transpose_kernel(const std::int32_t* __restrict__ order, 
 }
 
 // ---------------------------------------------------------------------------------------------
+// Columns scaled by dinv.
+// ---------------------------------------------------------------------------------------------
+__global__ void scale_columns_kernel(const std::int32_t* __restrict__ ci, const float* __restrict__ v,
+                                     const float* __restrict__ dinv, std::int64_t nnz, float* __restrict__ out) {
+    const std::int64_t p = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (p < nnz) out[p] = v[p] * dinv[ci[p]];
+}
+
+// ---------------------------------------------------------------------------------------------
 // Coarsest level: dense FP64 copy, then an in-place block Gauss-Jordan inverse (SPD: no pivoting).
 // ---------------------------------------------------------------------------------------------
 __global__ void csr_to_dense_kernel(const std::int32_t* __restrict__ rp, const std::int32_t* __restrict__ ci,
@@ -831,6 +840,15 @@ Cheby chebyshev(int degree, float lower_ratio) {
     return c;
 }
 
+void scale_columns(Level& L, hipStream_t s) {
+    L.scaled_val.reset(static_cast<std::size_t>(std::max<std::int64_t>(L.a.nnz, 1)), "scaled operator");
+    if (const unsigned g = grid_for(L.a.nnz))
+        scale_columns_kernel<<<g, kBlock, 0, s>>>(L.a.col, L.a.val, L.dinv.get(), L.a.nnz, L.scaled_val.get());
+    L.scaled = L.a;
+    L.scaled.val = L.scaled_val.get();
+    L.scaled.ell = nullptr;
+}
+
 // fem/solve.py:224-256 (aggregation_levels) and :259-284 (build_native_vcycle).
 Hierarchy build_hierarchy_like(const CsrView& a0, const Hierarchy& like, const AmgParams& prm, hipStream_t s) {
     if (like.levels.empty()) {  // the operator itself is the coarsest level
@@ -856,6 +874,7 @@ Hierarchy build_hierarchy_like(const CsrView& a0, const Hierarchy& like, const A
         }
         L.dinv.reset(static_cast<std::size_t>(L.a.n), "dinv");
         l1_dinv(L.a, L.dinv.get(), s);
+        scale_columns(L, s);
         L.p = smoothed_prolongator(L.a, ref.agg.get(), ref.n_coarse, L.dinv.get(), s);
         L.r = transpose(L.p.view(), s);
         L.n_coarse = ref.n_coarse;
@@ -888,6 +907,7 @@ Hierarchy build_hierarchy(const CsrView& a0, const AmgParams& prm, hipStream_t s
         }
         L.dinv.reset(static_cast<std::size_t>(L.a.n), "dinv");
         l1_dinv(L.a, L.dinv.get(), s);
+        scale_columns(L, s);
         L.p = smoothed_prolongator(L.a, agg.get(), nc, L.dinv.get(), s);
         L.r = transpose(L.p.view(), s);
         L.agg = std::move(agg);

@@ -100,7 +100,7 @@ struct cn_context {
     cn::DeviceBuffer<double> d_X, d_v, d_x0, d_rhs_sums;
     // Sliced ELL copies of the finest level's operator (with its diagonal, for the V-cycle) and of
     // the differenced off-diagonal operator (the block iteration's SpMM); width 0 when not built.
-    cn::DeviceBuffer<int2> ell_full, ell_off;
+    cn::DeviceBuffer<int2> ell_full, ell_scaled, ell_off;
     int ell_full_w = 0, ell_off_w = 0;
     // Missed-tolerance recovery counts: nominal hierarchy rebuilds, and preconditioners built for
     // one column's own operator (per-placement conductivities, conductivity draws).
@@ -114,6 +114,10 @@ struct cn_context {
             hier.levels[0].a.ell = max_k > 0 && ell_full_w > 0 ? ell_full.get() : nullptr;
             hier.levels[0].a.ell_w = ell_full_w;
             hier.levels[0].a.ell_max_k = max_k;
+            cn::CsrView& scaled = hier.levels[0].scaled;
+            scaled.ell = hier.levels[0].a.ell != nullptr ? ell_scaled.get() : nullptr;
+            scaled.ell_w = ell_full_w;
+            scaled.ell_max_k = max_k;
         }
         solver->set_off_ell(max_k > 0 && ell_off_w > 0 ? ell_off.get() : nullptr, ell_off_w, max_k);
     }
@@ -451,6 +455,7 @@ void build_context(cn_context& c, const double* nodes_mm, std::int64_t n, const 
     op.val64 = c.rval64.get();
     c.solver = std::make_unique<BlockSolver>(op, c.hier, s);
     c.ell_full_w = build_ell(c.reduced_view(), c.ell_full, s);
+    if (!c.hier.levels.empty()) build_ell(c.hier.levels[0].scaled, c.ell_scaled, s);
     c.ell_off_w = build_ell(op.off, c.ell_off, s);
     sync(s, "ell copies");
     lap();  // 7: differenced operator, solver, ELL copies

@@ -34,11 +34,15 @@ struct CsrView {
     int ell_max_k = 0;  // the row kernels take the ELL copy for block widths up to this
 };
 
-constexpr int kEllSlice = 64;
+// Eight rows: a slot's 64 bytes are one request whatever rows a wavefront holds. 64-row slices
+// measured 27.1 us where these take 22.7 (SpMM of four columns at 1.0M rows), and 46.8 against 36.0
+// at eight columns, whose wavefronts hold 16 rows.
+constexpr int kEllSlice = 8;
 // Widest block for which the sliced ELL copy is the default: at 1, 2 and 4 columns the row
 // kernels are bound by their index and value loads, which the ELL copy issues without waiting on
-// row pointers (the 1.5 mm head's plain solve: SpMM 34 -> 23 us, V-cycle 252 -> 209 us); at 8 and
-// 16 the gathers of whole W rows dominate and the CSR arrays measured as fast or faster.
+// row pointers (four columns at 1.0M rows: SpMM 34.3 -> 22.7 us, V-cycle 259 -> 222 us); at 8 and
+// 16 the gathers of whole W rows dominate and the CSR arrays measured as fast or faster (SpMM 35.4
+// against 36.0 us, 57.7 against 65.9).
 constexpr int kEllAutoMaxK = 4;
 constexpr int kEllMaxWidth = 24;  // rows longer than this keep the CSR kernels
 
@@ -77,6 +81,10 @@ struct Level {
     DeviceBuffer<float> dinv;
     DeviceBuffer<std::int32_t> agg;
     CsrF p, r;
+    // A with column j scaled by dinv_j (a's pattern): the smoother's pass from a zero guess reads it, so
+    // that pass gathers b alone and not dinv beside it (92 -> 83 us at 1.0M rows of 16 columns).
+    CsrView scaled;
+    DeviceBuffer<float> scaled_val;
     std::int64_t n_coarse = 0;
 };
 

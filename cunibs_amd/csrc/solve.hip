@@ -166,13 +166,10 @@ constexpr int gather_batch() {
     return SUB == 4 ? 4 : 8;
 }
 
-// With GS, the gathered rows are scaled on the fly: X_j -> (gs0 * gscale[j]) X_j (the Jacobi
-// iterate from zero, alpha0 dinv_j b_j, without writing it out).
-template <int K, int V, int SUB, bool DIFF, int U = gather_batch<SUB>(), bool GS = false>
+template <int K, int V, int SUB, bool DIFF, int U = gather_batch<SUB>()>
 __device__ __forceinline__ void row_gather_v(const std::int32_t* __restrict__ ci, const float* __restrict__ av, int j,
                                              int e, const float* __restrict__ X, int c0, const float (&xi)[V],
-                                             float (&acc)[V], const float* __restrict__ gscale = nullptr,
-                                             float gs0 = 0.0f) {
+                                             float (&acc)[V]) {
 #pragma unroll
     for (int v = 0; v < V; ++v) acc[v] = 0.0f;
     for (; j < e; j += U * SUB) {
@@ -187,23 +184,15 @@ __device__ __forceinline__ void row_gather_v(const std::int32_t* __restrict__ ci
             aa[u] = av[jj];
         }
         float xx[U][V];
-        float gw[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             vload<V>(X + static_cast<std::int64_t>(cc[u]) * K + c0, xx[u]);
-            if constexpr (GS) gw[u] = gscale[cc[u]];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float a = (j + u * SUB < e) ? aa[u] : 0.0f;
-            if constexpr (GS) {
-                const float w = gs0 * gw[u];
 #pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = fmaf(a, w * xx[u][v], acc[v]);
-            } else {
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = fmaf(a, DIFF ? xx[u][v] - xi[v] : xx[u][v], acc[v]);
-            }
+            for (int v = 0; v < V; ++v) acc[v] = fmaf(a, DIFF ? xx[u][v] - xi[v] : xx[u][v], acc[v]);
         }
     }
 }
@@ -240,11 +229,10 @@ __device__ __forceinline__ void row_gather_multi(const std::int32_t* __restrict_
 // (the row itself, value 0) adds an exact zero, so the sums are those of the CSR form. No row
 // pointers: the slot loads depend on nothing, and a wavefront's rows read one contiguous run per
 // slot.
-template <int K, int V, int SUB, bool DIFF, int U = gather_batch<SUB>(), bool GS = false>
+template <int K, int V, int SUB, bool DIFF, int U = gather_batch<SUB>()>
 __device__ __forceinline__ void ell_gather_v(const int2* __restrict__ pr, std::int64_t base, int j, int e,
                                              const float* __restrict__ X, int c0, const float (&xi)[V],
-                                             float (&acc)[V], const float* __restrict__ gscale = nullptr,
-                                             float gs0 = 0.0f) {
+                                             float (&acc)[V]) {
 #pragma unroll
     for (int v = 0; v < V; ++v) acc[v] = 0.0f;
     for (; j < e; j += U * SUB) {
@@ -258,23 +246,15 @@ __device__ __forceinline__ void ell_gather_v(const int2* __restrict__ pr, std::i
             aa[u] = __int_as_float(pv.y);
         }
         float xx[U][V];
-        float gw[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             vload<V>(X + static_cast<std::int64_t>(cc[u]) * K + c0, xx[u]);
-            if constexpr (GS) gw[u] = gscale[cc[u]];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float a = (j + u * SUB < e) ? aa[u] : 0.0f;
-            if constexpr (GS) {
-                const float w = gs0 * gw[u];
 #pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = fmaf(a, w * xx[u][v], acc[v]);
-            } else {
-#pragma unroll
-                for (int v = 0; v < V; ++v) acc[v] = fmaf(a, DIFF ? xx[u][v] - xi[v] : xx[u][v], acc[v]);
-            }
+            for (int v = 0; v < V; ++v) acc[v] = fmaf(a, DIFF ? xx[u][v] - xi[v] : xx[u][v], acc[v]);
         }
     }
 }
@@ -291,7 +271,8 @@ constexpr std::int64_t rows_per_vblock() {
 }
 
 enum RowMode : int {
-    kResidual = 0, kCheby = 1, kSpmm = 2, kSpmmDiff = 3, kSpmmDiffMulti = 4, kChebyZero = 5, kProlong = 6
+    kResidual = 0, kCheby = 1, kSpmm = 2, kSpmmDiff = 3, kSpmmDiffMulti = 4, kChebyZero = 5, kProlong = 6,
+    kPostFirst = 7, kPostLast = 8
 };
 
 // One kernel for every SpMV-shaped pass:
@@ -306,7 +287,11 @@ enum RowMode : int {
 //              updated in place by the row's own lanes)
 //   kChebyZero the first two smoothing steps from a zero guess in one pass: with
 //              x1 = alpha0 dinv b (formed on the fly for the row and its neighbours, never
-//              stored), out = c_cur x1 + alpha dinv (b - A x1); `x` is b and c_prev carries alpha0
+//              stored), out = c_cur x1 + alpha dinv (b - A x1); `x` is b, c_prev carries alpha0 and
+//              A's columns come scaled by dinv
+//   kPostFirst  out = x1 = alpha dinv (b - A x), the first correction after the coarse solution
+//   kPostLast  out = x_prev + c_cur x + alpha dinv A x, both steps' result from x = x1 (alpha is
+//              negative); out may alias x_prev
 // ELL: the rows come from the sliced ELL copy (ci holds its pairs, ell_w slots a row; rp and av
 // unused), the same sums as the CSR form.
 template <int K, int SUB, int MODE, bool ELL = false>
@@ -362,22 +347,19 @@ __global__ void __launch_bounds__(kRowThreads) rowk_kernel(
         float dg = 0.0f;
 #pragma unroll
         for (int v = 0; v < V; ++v) bb[v] = cur[v] = prev[v] = sv[v] = 0.0f;
-        if constexpr (MODE == kResidual || MODE == kCheby || MODE == kChebyZero) vload<V>(b + at, bb);
-        if constexpr (MODE == kCheby) {
+        if constexpr (MODE == kResidual || MODE == kCheby || MODE == kChebyZero || MODE == kPostFirst)
+            vload<V>(b + at, bb);
+        if constexpr (MODE == kCheby || MODE == kPostLast) {
             vload<V>(x + at, cur);
             vload<V>(x_prev + at, prev);
         }
         if constexpr (MODE == kProlong) vload<V>(x_prev + at, prev);  // out is x_prev
-        if constexpr (MODE == kCheby || MODE == kSpmmDiff || MODE == kChebyZero) dg = diag[rr];
+        if constexpr (MODE == kCheby || MODE == kSpmmDiff || MODE == kChebyZero || MODE == kPostFirst || MODE == kPostLast)
+            dg = diag[rr];
         if constexpr (MODE == kSpmmDiffMulti) vload<V>(diag + at, sv);
         if constexpr (MODE == kSpmmDiffMulti) {
             static_assert(!ELL, "the multi-matrix values follow the CSR entries");
             row_gather_multi<K, V, SUB>(ci, av, j0, e, x, c0, xi, acc);
-        } else if constexpr (MODE == kChebyZero) {
-            if constexpr (ELL)
-                ell_gather_v<K, V, SUB, false, gather_batch<SUB>(), true>(pr, ebase, j0, e, x, c0, xi, acc, diag, c_prev);
-            else
-                row_gather_v<K, V, SUB, false, gather_batch<SUB>(), true>(ci, av, j0, e, x, c0, xi, acc, diag, c_prev);
         } else {
             if constexpr (ELL)
                 ell_gather_v<K, V, SUB, MODE == kSpmmDiff>(pr, ebase, j0, e, x, c0, xi, acc);
@@ -410,8 +392,16 @@ __global__ void __launch_bounds__(kRowThreads) rowk_kernel(
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 const float x1 = w * bb[v];
-                o[v] = fmaf(d, bb[v] - acc[v], fmaf(0.0f, x1, c_cur * x1));
+                o[v] = fmaf(d, fmaf(-c_prev, acc[v], bb[v]), c_cur * x1);
             }
+        } else if constexpr (MODE == kPostFirst) {
+            const float d = alpha * dg;
+#pragma unroll
+            for (int v = 0; v < V; ++v) o[v] = d * (bb[v] - acc[v]);
+        } else if constexpr (MODE == kPostLast) {
+            const float d = alpha * dg;
+#pragma unroll
+            for (int v = 0; v < V; ++v) o[v] = prev[v] + fmaf(d, acc[v], c_cur * cur[v]);
         } else {
             const float d = alpha * dg;
 #pragma unroll
@@ -1639,7 +1629,7 @@ void run_vcycle(const Hierarchy& h, const std::vector<int>& subs, std::vector<De
             // Jacobi from zero and the Chebyshev step after it, in one pass (the Jacobi iterate is
             // only ever read by that step).
             float* out = target(1);
-            launch_rows<K, kChebyZero>(sub, L.a, L.dinv.get(), bi, bi, nullptr, ch.c_cur[0], ch.alpha0, ch.alpha[0],
+            launch_rows<K, kChebyZero>(sub, L.scaled, L.dinv.get(), bi, bi, nullptr, ch.c_cur[0], ch.alpha0, ch.alpha[0],
                                        out, state, s);
             return out;
         }
@@ -1687,7 +1677,20 @@ void run_vcycle(const Hierarchy& h, const std::vector<int>& subs, std::vector<De
         const CsrView P = L.p.view();
         launch_rows<K, kProlong>(choose_sub(P.n, P.nnz, col_groups<K>(), n_cu), P, nullptr, nullptr, xc, lx[i].get(),
                                  0.f, 0.f, 0.f, lx[i].get(), state, s);
-        xc = smooth(i, bi, lx[i].get(), lr[i].get(), lx[i].get(), (i == first) ? X : nullptr);
+        float* const out = i == first ? X : lx[i].get();
+        if (ch.degree == 2) {
+            // Both steps in terms of the first one's correction x1 = alpha0 dinv (b - A x): with
+            // c_cur + c_prev = 1 the second is x + (c_cur + alpha / alpha0) x1 - alpha dinv A x1, which
+            // reads neither b nor a second iterate (96 + 96 us as two general steps at 1.0M rows of 16
+            // columns, 83 + 87 so; both move about 330 MB, 4 TB/s with the gather).
+            launch_rows<K, kPostFirst>(subs[i], L.a, L.dinv.get(), bi, lx[i].get(), nullptr, 0.f, 0.f, ch.alpha0,
+                                       lr[i].get(), state, s);
+            launch_rows<K, kPostLast>(subs[i], L.a, L.dinv.get(), nullptr, lr[i].get(), lx[i].get(),
+                                      ch.c_cur[0] + ch.alpha[0] / ch.alpha0, 0.f, -ch.alpha[0], out, state, s);
+            xc = out;
+        } else {
+            xc = smooth(i, bi, lx[i].get(), lr[i].get(), lx[i].get(), (i == first) ? X : nullptr);
+        }
     }
 }
 
