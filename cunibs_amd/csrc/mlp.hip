@@ -2,8 +2,9 @@
 // trained on the GPU with the library's own kernels, mapping a placement's pose (and tissue
 // conductivities) to coefficients in the reduced basis of solver-generated solutions.
 //
-// Training runs in FP32: tiled GEMMs on the vector ALUs for the forward pass, the backward pass and
-// the weight gradients, an exact GELU (erf form) and Adam on FP32 master weights. Inference uses
+// Training runs in FP32: GEMMs on the FP32 matrix cores for the forward pass, the backward pass and
+// the weight gradients, with the bias, an exact GELU (erf form), its derivative and the bias gradient
+// in the same kernels, and Adam on FP32 master weights. Inference uses
 // BF16 copies of the weights: each layer is a v_mfma_f32_16x16x16bf16_1k GEMM with FP32
 // accumulation, the activations rounded to BF16 between layers.
 //
@@ -19,59 +20,8 @@ namespace cn {
 
 namespace {
 
-constexpr int kTile = 64;   // output tile of the FP32 GEMM (64 x 64 per 256-thread block)
-constexpr int kTileK = 16;  // K chunk staged in LDS
-
-// C[i, j] = (accumulate ? C[i, j] : 0) + sum_k A(i, k) B(k, j) (+ bias[j]), FP32. A(i, k) is
-// A[i * sa_i + k * sa_k] and B(k, j) is B[k * sb_k + j * sb_j], so transposed operands are strides.
-// Each thread owns a 4 x 4 block of the tile; k runs in ascending order for every output.
-__global__ void __launch_bounds__(256) gemm_f32_kernel(int M, int N, int K, const float* __restrict__ A,
-                                                       long sa_i, long sa_k, const float* __restrict__ B, long sb_k,
-                                                       long sb_j, float* __restrict__ C, int ldc,
-                                                       const float* __restrict__ bias, int accumulate) {
-    __shared__ float As[kTileK][kTile + 1];
-    __shared__ float Bs[kTileK][kTile + 1];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int i0 = blockIdx.y * kTile, j0 = blockIdx.x * kTile;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += kTileK) {
-        for (int e = threadIdx.x; e < kTileK * kTile; e += 256) {
-            const int kk = e / kTile, r = e % kTile;
-            const int i = i0 + r, j = j0 + r, k = k0 + kk;
-            As[kk][r] = (i < M && k < K) ? A[i * sa_i + k * sa_k] : 0.0f;
-            Bs[kk][r] = (j < N && k < K) ? B[k * sb_k + j * sb_j] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < kTileK; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a[u] = As[kk][ty * 4 + u];
-                b[u] = Bs[kk][tx * 4 + u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[u][v] = fmaf(a[u], b[v], acc[u][v]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int i = i0 + ty * 4 + u;
-        if (i >= M) continue;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int j = j0 + tx * 4 + v;
-            if (j >= N) continue;
-            float r = acc[u][v];
-            if (bias) r += bias[j];
-            if (accumulate) r += C[static_cast<long>(i) * ldc + j];
-            C[static_cast<long>(i) * ldc + j] = r;
-        }
-    }
-}
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4_t;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -79,16 +29,150 @@ __device__ __forceinline__ float gelu_grad(float x) {
     return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
 }
 
-__global__ void gelu_kernel(long count, const float* __restrict__ z, float* __restrict__ h) {
-    const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < count) h[i] = gelu(z[i]);
+constexpr int kTile = 64;    // output tile of the FP32 GEMM: 64 x 64 per block, 32 x 32 per wavefront
+constexpr int kTileK = 32;   // K chunk staged in LDS
+constexpr int kPitch = kTileK + 4;
+constexpr int kGemmThreads = 256;
+
+enum Epilogue : int {
+    kPlain = 0,     // C = acc
+    kBias = 1,      // C = acc + bias
+    kGelu = 2,      // C = z = acc + bias, H = gelu(z)
+    kGeluGrad = 3,  // C = acc gelu'(Z)
+};
+
+struct GemmArgs {
+    int M, N, K;
+    const float* A;  // A(i, k): A[i * lda + k], or A[k * lda + i] transposed
+    int lda;
+    const float* B;  // B(k, j): B[k * ldb + j], or B[j * ldb + k] transposed
+    int ldb;
+    float* C;  // (M, N), the split's part of the partials when K is split
+    const float* bias;
+    const float* Z;
+    float* H;
+    float* colsum;  // kPlain: column sums of B over its K rows (the bias gradient)
+    int k_per;      // K rows per split, a multiple of kTileK (blockIdx.z = split)
+};
+
+// One operand's 64 x kTileK chunk into registers: two float4 a thread along the contiguous dimension
+// (leading dimensions and contiguous extents are multiples of 4), zeros past the edges.
+// KC: k is contiguous. `r` counts rows of the tile, `R` the extent of that dimension.
+template <bool KC>
+__device__ __forceinline__ void load_chunk(const float* __restrict__ p, int ld, int r0, int R, int k0, int k1,
+                                           float4 (&v)[2]) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int t = threadIdx.x + u * kGemmThreads;
+        const int r = r0 + (KC ? t / (kTileK / 4) : 4 * (t % (kTile / 4)));
+        const int k = k0 + (KC ? 4 * (t % (kTileK / 4)) : t / (kTile / 4));
+        v[u] = (r < R && k < k1) ? *reinterpret_cast<const float4*>(p + (KC ? static_cast<long>(r) * ld + k
+                                                                             : static_cast<long>(k) * ld + r))
+                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
 }
 
-// dz = dh * gelu'(z)
-__global__ void gelu_back_kernel(long count, const float* __restrict__ z, const float* __restrict__ dh,
-                                 float* __restrict__ dz) {
+// The chunk into LDS as rows of kTileK consecutive k.
+template <bool KC>
+__device__ __forceinline__ void store_chunk(const float4 (&v)[2], float (&s)[kTile][kPitch]) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int t = threadIdx.x + u * kGemmThreads;
+        if constexpr (KC) {
+            *reinterpret_cast<float4*>(&s[t / (kTileK / 4)][4 * (t % (kTileK / 4))]) = v[u];
+        } else {
+            const int r = 4 * (t % (kTile / 4)), k = t / (kTile / 4);
+            s[r][k] = v[u].x;
+            s[r + 1][k] = v[u].y;
+            s[r + 2][k] = v[u].z;
+            s[r + 3][k] = v[u].w;
+        }
+    }
+}
+
+// C = A B on the FP32 matrix cores (v_mfma_f32_16x16x4f32, FP32 products and sums). Each wavefront
+// keeps 2 x 2 tiles of 16 x 16; a lane reads four consecutive k of its row of either operand in one
+// 16-byte LDS read and feeds them to four products, so product u of a 16-k group takes the k's
+// 4 (l / 16) + u of both. The next chunk's global loads are in flight during the products.
+// The weight gradients have few tiles (64 for 512 x 512) and a long K, so they split K over
+// blockIdx.z until 512 blocks are in flight, partials added in order. The gradients of a 2048-row
+// batch at 512 hidden and 256 outputs: 3.4 ms with vector-ALU tiles, unsplit, and a bias gradient
+// serial in the rows; 0.7 ms now with the copies, 0.16 ms of it in these kernels (24 us for the
+// 2048 x 512 x 512 product, 45 TFLOP/s: its 256 blocks are one wavefront a SIMD).
+template <bool AKC, bool BKC, int EPI>
+__global__ void __launch_bounds__(kGemmThreads) gemm_f32_kernel(GemmArgs g) {
+    __shared__ __align__(16) float As[kTile][kPitch];
+    __shared__ __align__(16) float Bs[kTile][kPitch];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row = lane & 15, quad = lane >> 4;
+    const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1);
+    const int i0 = blockIdx.y * kTile, j0 = blockIdx.x * kTile;
+    const int k0 = blockIdx.z * g.k_per, k1 = min(k0 + g.k_per, g.K);
+    floatx4_t acc[2][2] = {};
+    float sum = 0.0f;
+    float4 av[2], bv[2];
+    load_chunk<AKC>(g.A, g.lda, i0, g.M, k0, k1, av);
+    load_chunk<BKC>(g.B, g.ldb, j0, g.N, k0, k1, bv);
+    for (int k = k0; k < k1; k += kTileK) {
+        store_chunk<AKC>(av, As);
+        store_chunk<BKC>(bv, Bs);
+        __syncthreads();
+        load_chunk<AKC>(g.A, g.lda, i0, g.M, k + kTileK, k1, av);
+        load_chunk<BKC>(g.B, g.ldb, j0, g.N, k + kTileK, k1, bv);
+#pragma unroll
+        for (int c = 0; c < kTileK; c += 16) {
+            floatx4_t a[2], b[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                a[x] = *reinterpret_cast<const floatx4_t*>(&As[wi + 16 * x + row][c + 4 * quad]);
+                b[x] = *reinterpret_cast<const floatx4_t*>(&Bs[wj + 16 * x + row][c + 4 * quad]);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x][u], b[y][u], acc[x][y], 0, 0, 0);
+        }
+        if constexpr (EPI == kPlain) {
+            if (g.colsum != nullptr && blockIdx.y == 0 && threadIdx.x < kTile)
+                for (int kk = 0; kk < kTileK; ++kk) sum += Bs[threadIdx.x][kk];
+        }
+        __syncthreads();
+    }
+    const long part = static_cast<long>(blockIdx.z) * g.M * g.N;
+    if constexpr (EPI == kPlain) {
+        if (g.colsum != nullptr && blockIdx.y == 0 && threadIdx.x < kTile && j0 + static_cast<int>(threadIdx.x) < g.N)
+            g.colsum[static_cast<long>(blockIdx.z) * g.N + j0 + threadIdx.x] = sum;
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = i0 + wi + 16 * x + 4 * quad + v, j = j0 + wj + 16 * y + row;
+                if (i >= g.M || j >= g.N) continue;
+                const long at = static_cast<long>(i) * g.N + j;
+                float r = acc[x][y][v];
+                if constexpr (EPI == kBias || EPI == kGelu) r += g.bias[j];
+                if constexpr (EPI == kGeluGrad) r *= gelu_grad(g.Z[at]);
+                g.C[part + at] = r;
+                if constexpr (EPI == kGelu) g.H[at] = gelu(r);
+            }
+}
+
+// out = the splits' partials added in order: the product's `count` values, then the bias gradient's N.
+__global__ void sum_splits_kernel(long count, int N, int splits, const float* __restrict__ parts,
+                                  const float* __restrict__ cols, float* __restrict__ out, float* __restrict__ db) {
     const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < count) dz[i] = dh[i] * gelu_grad(z[i]);
+    if (i >= count + N) return;
+    const float* p = i < count ? parts + i : cols + (i - count);
+    const long step = i < count ? count : N;
+    float acc = p[0];
+    for (int z = 1; z < splits; ++z) acc += p[z * step];
+    (i < count ? out[i] : db[i - count]) = acc;
 }
 
 // Mean squared error over the batch: dy = 2 (y - t) / (B * N); per-row partial losses in FP64.
@@ -109,15 +193,6 @@ __global__ void mse_kernel(int B, int N, const float* __restrict__ y, const floa
         __syncthreads();
     }
     if (threadIdx.x == 0) row_loss[r] = s[0];
-}
-
-// Bias gradient: db[j] = sum over rows of dz[r, j], rows in order.
-__global__ void bias_grad_kernel(int B, int N, const float* __restrict__ dz, float* __restrict__ db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
-    float acc = 0.0f;
-    for (int r = 0; r < B; ++r) acc += dz[static_cast<long>(r) * N + j];
-    db[j] = acc;
 }
 
 __device__ __forceinline__ unsigned short to_bf16(float x) {
@@ -145,9 +220,6 @@ __global__ void to_bf16_kernel(long count, const float* __restrict__ x, unsigned
     const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < count) y[i] = to_bf16(x[i]);
 }
-
-typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4_t;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 
 // Y (M, N) FP32 = act(X (M, K) BF16 . W (K, N) BF16 + bias), one wavefront per 16 x 16 tile,
 // K stepped by 16 (M, N, K multiples of 16). Lane l supplies A[l % 16][4 (l / 16) + j],
@@ -184,10 +256,18 @@ __global__ void __launch_bounds__(256) mfma_layer_kernel(int M, int N, int K, co
     }
 }
 
-void gemm(int M, int N, int K, const float* A, long sa_i, long sa_k, const float* B, long sb_k, long sb_j, float* C,
-          int ldc, const float* bias, bool accumulate, hipStream_t s) {
-    const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
-    gemm_f32_kernel<<<grid, 256, 0, s>>>(M, N, K, A, sa_i, sa_k, B, sb_k, sb_j, C, ldc, bias, accumulate ? 1 : 0);
+template <bool AKC, bool BKC, int EPI>
+void gemm(GemmArgs g, int splits, hipStream_t s) {
+    const int chunks = (g.K + kTileK - 1) / kTileK;
+    g.k_per = (chunks + splits - 1) / splits * kTileK;
+    const dim3 grid((g.N + kTile - 1) / kTile, (g.M + kTile - 1) / kTile, splits);
+    gemm_f32_kernel<AKC, BKC, EPI><<<grid, kGemmThreads, 0, s>>>(g);
+}
+
+// Splits of the batch in a weight gradient: until 512 blocks are in flight, each of at least 256 rows.
+int grad_splits(int M, int N, int B) {
+    const int tiles = ((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile);
+    return std::max(1, std::min({512 / tiles, B / 256, 64}));
 }
 
 }  // namespace
@@ -244,8 +324,14 @@ void Mlp::ensure_batch(int B) {
     y_.reset(static_cast<long>(B) * n_out_, "y");
     t_.reset(static_cast<long>(B) * n_out_, "t");
     dy_.reset(static_cast<long>(B) * n_out_, "dy");
-    dh_.reset(hb, "dh");
     dz_.reset(hb, "dz");
+    dz1_.reset(hb, "dz1");
+    const int shapes[3][2] = {{kInPad, n_hidden_}, {n_hidden_, n_hidden_}, {n_hidden_, n_out_}};
+    std::size_t parts = 1;  // at most 512 tiles of partials; a smaller batch splits no further
+    for (const auto& m : shapes)
+        if (const int z = grad_splits(m[0], m[1], B); z > 1)
+            parts = std::max(parts, static_cast<std::size_t>(z) * (m[0] + 1) * m[1]);
+    parts_.reset(parts, "gradient partials");
     loss_.reset(B, "row loss");
     x16_.reset(static_cast<long>(B) * kInPad, "x16");
     h16a_.reset(hb, "h16a");
@@ -272,26 +358,34 @@ double Mlp::forward_backward(int B) {
     const float* b2 = w_.get() + boffset_[1];
     const float* W3 = w_.get() + offset_[2];
     const float* b3 = w_.get() + boffset_[2];
-    const long hb = static_cast<long>(B) * H;
     // forward
-    gemm(B, H, kInPad, x_.get(), kInPad, 1, W1, H, 1, z1_.get(), H, b1, false, s_);
-    gelu_kernel<<<grid_for(hb), kBlock, 0, s_>>>(hb, z1_.get(), h1_.get());
-    gemm(B, H, H, h1_.get(), H, 1, W2, H, 1, z2_.get(), H, b2, false, s_);
-    gelu_kernel<<<grid_for(hb), kBlock, 0, s_>>>(hb, z2_.get(), h2_.get());
-    gemm(B, O, H, h2_.get(), H, 1, W3, O, 1, y_.get(), O, b3, false, s_);
+    gemm<true, false, kGelu>({B, H, kInPad, x_.get(), kInPad, W1, H, z1_.get(), b1, nullptr, h1_.get()}, 1, s_);
+    gemm<true, false, kGelu>({B, H, H, h1_.get(), H, W2, H, z2_.get(), b2, nullptr, h2_.get()}, 1, s_);
+    gemm<true, false, kBias>({B, O, H, h2_.get(), H, W3, O, y_.get(), b3}, 1, s_);
     mse_kernel<<<B, 256, 0, s_>>>(B, O, y_.get(), t_.get(), dy_.get(), loss_.get());
-    // backward: dW3 = h2^T dy, db3, dh2 = dy W3^T, dz2, dW2 = h1^T dz2, ...
+    // backward: dW3 = h2^T dy and db3, dz2 = (dy W3^T) gelu'(z2), dW2 = h1^T dz2, ...
     float* G = g_.get();
-    gemm(H, O, B, h2_.get(), 1, H, dy_.get(), O, 1, G + offset_[2], O, nullptr, false, s_);
-    bias_grad_kernel<<<grid_for(O), kBlock, 0, s_>>>(B, O, dy_.get(), G + boffset_[2]);
-    gemm(B, H, O, dy_.get(), O, 1, W3, 1, O, dh_.get(), H, nullptr, false, s_);
-    gelu_back_kernel<<<grid_for(hb), kBlock, 0, s_>>>(hb, z2_.get(), dh_.get(), dz_.get());
-    gemm(H, H, B, h1_.get(), 1, H, dz_.get(), H, 1, G + offset_[1], H, nullptr, false, s_);
-    bias_grad_kernel<<<grid_for(H), kBlock, 0, s_>>>(B, H, dz_.get(), G + boffset_[1]);
-    gemm(B, H, H, dz_.get(), H, 1, W2, 1, H, dh_.get(), H, nullptr, false, s_);
-    gelu_back_kernel<<<grid_for(hb), kBlock, 0, s_>>>(hb, z1_.get(), dh_.get(), dz_.get());
-    gemm(kInPad, H, B, x_.get(), 1, kInPad, dz_.get(), H, 1, G + offset_[0], H, nullptr, false, s_);
-    bias_grad_kernel<<<grid_for(H), kBlock, 0, s_>>>(B, H, dz_.get(), G + boffset_[0]);
+    auto weight_grad = [&](int M, int N, const float* in, const float* d, int l) {
+        const int splits = grad_splits(M, N, B);
+        GemmArgs a{M, N, B, in, M, d, N, G + offset_[l]};
+        a.colsum = G + boffset_[l];
+        if (splits == 1) {
+            gemm<false, false, kPlain>(a, 1, s_);
+            return;
+        }
+        const long count = static_cast<long>(M) * N;
+        a.C = parts_.get();
+        a.colsum = parts_.get() + splits * count;
+        gemm<false, false, kPlain>(a, splits, s_);
+        sum_splits_kernel<<<grid_for(count + N), kBlock, 0, s_>>>(count, N, splits, parts_.get(), a.colsum,
+                                                                  G + offset_[l], G + boffset_[l]);
+    };
+    weight_grad(H, O, h2_.get(), dy_.get(), 2);
+    gemm<true, true, kGeluGrad>({B, H, O, dy_.get(), O, W3, O, dz_.get(), nullptr, z2_.get()}, 1, s_);
+    weight_grad(H, H, h1_.get(), dz_.get(), 1);
+    gemm<true, true, kGeluGrad>({B, H, H, dz_.get(), H, W2, H, dz1_.get(), nullptr, z1_.get()}, 1, s_);
+    weight_grad(kInPad, H, x_.get(), dz1_.get(), 0);
+    check(hipGetLastError(), "mlp launches");
     std::vector<double> rl(B);
     d2h(rl.data(), loss_.get(), B, s_);
     sync(s_, "mlp step");

@@ -35,7 +35,8 @@ class Mlp {
     int cap_batch_ = 0;
     DeviceBuffer<float> w_, g_, m_, v_;
     DeviceBuffer<unsigned short> w16_;
-    DeviceBuffer<float> x_, z1_, h1_, z2_, h2_, y_, t_, dy_, dh_, dz_;
+    DeviceBuffer<float> x_, z1_, h1_, z2_, h2_, y_, t_, dy_, dz_, dz1_;
+    DeviceBuffer<float> parts_;  // weight gradients' partials over splits of the batch
     DeviceBuffer<double> loss_;
     PinnedStage stage_;  // padded inputs, copied without a wait
     DeviceBuffer<unsigned short> x16_, h16a_, h16b_;

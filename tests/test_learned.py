@@ -48,6 +48,27 @@ def test_gpu_gradients_match_the_oracle(oracle_mod):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch,hidden,n_out", [(1, 16, 16), (63, 64, 48), (65, 80, 16), (255, 16, 144), (511, 64, 64),
+                                                (515, 144, 80), (2049, 80, 48)])
+def test_gpu_gradients_at_tile_and_split_edges(oracle_mod, batch, hidden, n_out):
+    """Ragged rows and columns of the 64 x 64 tiles, K chunks cut short, and batches at both sides of
+    the splits of the weight gradients (256 rows each, the last one partly or wholly empty)."""
+    from cunibs_amd.learned import WarmStartNetwork
+    net = WarmStartNetwork(n_out=n_out, hidden=hidden, seed=3, n_in=14)
+    rng = np.random.default_rng(batch)
+    X = rng.normal(size=(batch, 14)).astype(np.float32)
+    T = rng.normal(size=(batch, n_out)).astype(np.float32)
+    p = net.params()
+    loss, g = net.gradients(X, T)
+    want_loss, want = oracle_mod.mlp_loss_and_gradients(p.astype(np.float64), X.astype(np.float64),
+                                                        T.astype(np.float64), hidden, n_out)
+    # A gradient passes through sums of hidden, hidden, n_out and batch FP32 terms: n eps each at worst.
+    bound = 2.0 ** -24 * (batch + 2 * hidden + n_out + 64)
+    assert loss == pytest.approx(want_loss, rel=bound)
+    assert np.linalg.norm(g - want) <= bound * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
 def test_gpu_bf16_inference_matches_an_emulation(oracle_mod):
     from cunibs_amd.learned import WarmStartNetwork
     net = WarmStartNetwork(n_out=32, hidden=64, seed=4, n_in=14)
