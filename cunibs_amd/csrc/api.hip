@@ -17,6 +17,7 @@
 #include "prims.hpp"
 #include "recovery.hpp"
 #include "mlp.hpp"
+#include "output_copy.hpp"
 #include "uq.hpp"
 #include "warm.hpp"
 #include "solve.hpp"
@@ -121,6 +122,8 @@ struct cn_context {
         }
         solver->set_off_ell(max_k > 0 && ell_off_w > 0 ? ell_off.get() : nullptr, ell_off_w, max_k);
     }
+    // Fields on their way to the caller's arrays.
+    cn::OutputCopy out_copy;
     // The nodes' boxes and the current call's coil, for the N-body (dipole.hip).
     cn::BoxTree boxes;
     cn::DipoleSet dipoles;
@@ -902,8 +905,7 @@ void uq_solve(cn_context& c, const double* sigma, int k, const cn_solve_options*
         auto fetch = [&](float* host, const float* dev, std::int64_t rows, int inner) {
             c.d_stage.ensure(rows * inner * k, "output staging");
             unpack(dev, rows, inner, k, K, c.d_stage.get(), s);
-            d2h(host, c.d_stage.get(), rows * inner * k, s);
-            sync(s, "output copy");
+            c.out_copy.run(host, c.d_stage.get(), sizeof(float) * rows * inner * k, s);
         };
         if (out->transforms)
             for (int i = 0; i < k; ++i) std::memcpy(out->transforms + 16 * i, u.transform, sizeof(double) * 16);
@@ -912,7 +914,7 @@ void uq_solve(cn_context& c, const double* sigma, int k, const cn_solve_options*
         if (out->v) {
             c.d_v.ensure(n * k, "potential");
             scatter_potential(c.d_X.get(), n, k, K, c.ground, c.d_v.get(), s);
-            d2h(out->v, c.d_v.get(), n * k, s);
+            c.out_copy.run(out->v, c.d_v.get(), sizeof(*out->v) * n * k, s);
         }
         if (out->metrics)
             region_metrics(c.d_magn.get(), m, k, K, c.region_idx.get(), c.n_region, c.vols32.get(), c.bary.get(),
@@ -1139,8 +1141,7 @@ void solve_block(cn_context& c, const double* pos_m, const double* mom, std::int
         auto fetch = [&](float* host, const float* dev, std::int64_t rows, int inner) {
             c.d_stage.ensure(rows * inner * k, "output staging");
             unpack(dev, rows, inner, k, K, c.d_stage.get(), s);
-            d2h(host, c.d_stage.get(), rows * inner * k, s);
-            sync(s, "output copy");
+            c.out_copy.run(host, c.d_stage.get(), sizeof(float) * rows * inner * k, s);
         };
         if (out->magnE) fetch(out->magnE, c.d_magn.get(), m, 1);
         if (out->E) fetch(out->E, c.d_E.get(), m, 3);
@@ -1150,11 +1151,11 @@ void solve_block(cn_context& c, const double* pos_m, const double* mom, std::int
         }
         if (out->dadt_elm) fetch(out->dadt_elm, c.d_dadt_elm.get(), m, 3);
         if (out->dadt_nodes) fetch(out->dadt_nodes, c.d_dadt_nodes.get(), n, 3);
-        if (out->rhs) d2h(out->rhs, c.d_rhs.get(), n * k, s);
+        if (out->rhs) c.out_copy.run(out->rhs, c.d_rhs.get(), sizeof(*out->rhs) * n * k, s);
         if (out->v) {
             c.d_v.ensure(n * k, "potential");
             scatter_potential(c.d_X.get(), n, k, K, c.ground, c.d_v.get(), s);
-            d2h(out->v, c.d_v.get(), n * k, s);
+            c.out_copy.run(out->v, c.d_v.get(), sizeof(*out->v) * n * k, s);
         }
         if (out->metrics)
             region_metrics(c.d_magn.get(), m, k, K, c.region_idx.get(), c.n_region, c.vols32.get(), c.bary.get(),

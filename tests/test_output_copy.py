@@ -1,0 +1,34 @@
+"""Fields copied through the ring of pinned chunks (csrc/output_copy.hpp) against those below its
+smallest size: the norm of E, element by element, is the |E| of the same block."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cunibs_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from cunibs_amd import fem
+    head = synthetic.shell_head(4.0, perturb_rms_mm=1.0, seed=2)
+    c = fem.SolverContext(head.nodes_mm, head.tet_nodes, head.tet_tags, head.skin_tris)
+    yield c
+    c.free()
+
+
+@pytest.mark.parametrize("k", [1, 2, 4, 5])  # E of 3.7, 7.4, 14.9 and 18.6 MB: below the ring, within it, past it
+def test_fields_through_the_ring(ctx, k):
+    from cunibs_amd import fem
+    coil = synthetic.figure8_coil(seed=3, per_layer=40)
+    sites = synthetic.cap_sites(k, seed=k)
+    res = fem.solve_placements_block(ctx, coil.positions_m, coil.moments, sites, 1e6, vectors=True, potential=True,
+                                     tolerance=0.5)
+    for r in res:
+        norm = np.linalg.norm(r.E.astype(np.float64), axis=1)
+        # three FP32 products and sums and a square root: 4 eps
+        assert np.all(np.abs(norm - r.magnE) <= 4 * 2.0 ** -24 * norm + 1e-30)
+        assert np.all(np.isfinite(r.v))
