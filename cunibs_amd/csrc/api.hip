@@ -873,6 +873,7 @@ void uq_solve(cn_context& c, const double* sigma, int k, const cn_solve_options*
         sync(s, "uq initial guess");
         dx0 = c.d_x0.get();
     }
+    opt.take_constant = out != nullptr && out->v != nullptr;
     c.solver->set_multi(&u.mop);
     SolveStats st;
     try {

@@ -2249,7 +2249,7 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
             sync(s_, "right-hand-side norms");
             check_bnorm();
         }
-        {  // the constant part of the error, and the solution handed out
+        if (opt.take_constant) {  // the constant part of the error, and the solution handed out
             const std::int64_t blocks = (nn + kWave - 1) / kWave;
             constexpr int kSumThreads = kWave * K < 1024 ? kWave * K : 1024;
             double* const shift = shift_.get();
@@ -2280,7 +2280,7 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
         true_residual(false);
         bool over = false;
         for (int c = 0; c < k; ++c) over |= !(rnorm[c] <= opt.tolerance * bnorm[c]);
-        if (over) {
+        if (over && handed_out) {
             undo_shift_kernel<<<1, kWave, 0, s_>>>(K, opt.tolerance, norms_.get(), bnorm_.get(), shift_.get());
             shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift_.get(), Xi, X);
             true_residual(false);
