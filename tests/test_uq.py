@@ -65,6 +65,39 @@ def test_uq_samples_match_per_sample_fp64_solves(head4, coil, oracle_mod):
 
 
 @pytest.mark.gpu
+def test_placements_prepared_anew_keep_the_captured_iterations(head8, coil):
+    """A second placement's draws replay the iterations captured for the first's, whatever was allocated
+    in between, and give what a context of their own gives."""
+    from cunibs_amd import fem, synthetic, uq
+    mesh = (head8.nodes_mm, head8.tet_nodes, head8.tet_tags, head8.skin_tris)
+    sites = synthetic.cap_sites(3, seed=29)
+
+    def draws(ctx, site):
+        tags = ctx.uq_prepare(coil.positions_m, coil.moments, site, 1e6)
+        sigma = uq.draw_lognormal(tags, 11, 0.2, seed=2)
+        fields = [r.magnE for part in (sigma[:8], sigma[8:]) for r in ctx.uq_solve(part)]
+        return np.stack(fields), ctx.uq_moments()
+
+    ctx, others = fem.SolverContext(*mesh), []
+    try:
+        draws(ctx, sites[0])  # every width's buffers and captures, the single-column solve's second ones
+        draws(ctx, sites[0])
+        count = ctx.graph_execs()
+        for site in sites:
+            fields, (mean, var, n) = draws(ctx, site)
+            assert ctx.graph_execs() == count
+            assert n == 11
+            others.append(fem.SolverContext(*mesh))  # takes the memory that the placement gave back
+            want, (want_mean, want_var, _) = draws(others[-1], site)
+            np.testing.assert_array_equal(fields, want)
+            np.testing.assert_array_equal(mean, want_mean)
+            np.testing.assert_array_equal(var, want_var)
+    finally:
+        for c in (ctx, *others):
+            c.free()
+
+
+@pytest.mark.gpu
 def test_per_placement_conductivities_match_fp64_solves(head4, coil, oracle_mod):
     """solve_placements_block(sigma=...): every placement of a block with its own conductivities,
     against the FP64 oracle built with that placement's table; the nominal row reproduces the
