@@ -71,6 +71,8 @@ struct cn_context {
     cn_options opts{};
     std::int64_t n = 0, m = 0, n_skin = 0;
     int ground = 0;
+    cn::DeviceBuffer<std::int32_t> ground_rows;  // reduced rows of the ground's neighbours
+    int n_ground = 0;
     int n_cu = 256;
     cn::DeviceBuffer<double> nodes, bary, skin_a, skin_b, skin_c, skin_n;
     cn::DeviceBuffer<std::int32_t> tets, tags, skin, node_perm, tet_perm;
@@ -263,6 +265,18 @@ __global__ void region_volume_kernel(const std::int32_t* __restrict__ idx, std::
     if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
+// The neighbours of the ground node (its row's other columns), as rows of the reduced operator.
+__global__ void ground_rows_kernel(const std::int32_t* __restrict__ rp, const std::int32_t* __restrict__ ci, int ground,
+                                   std::int32_t* __restrict__ rows) {
+    const int b = rp[ground], e = rp[ground + 1];
+    int at = 0;  // the ground's own entry in its row (the row is empty if no tetrahedron has the node)
+    while (at < e - b && ci[b + at] != ground) ++at;
+    for (int i = threadIdx.x; i < e - b; i += cn::kWave) {
+        const int j = ci[b + i];
+        if (i != at) rows[i - (i > at)] = j - (j > ground);
+    }
+}
+
 // Row r of the differenced operator: its off-diagonal entries in order, and the FP64 row sum
 // (diagonal included) rounded once to FP32.
 __global__ void offdiag_kernel(const std::int32_t* __restrict__ rp, const std::int32_t* __restrict__ ci,
@@ -414,6 +428,9 @@ void build_context(cn_context& c, const double* nodes_mm, std::int64_t n, const 
     c.ground = lowest_z_node(c.nodes.get(), n, s);
     c.nnz_red = reduce_grounded(indptr.get(), indices.get(), data.get(), n, c.ground, c.rptr, c.rcol, c.rval64,
                                 c.rval32, s);
+    c.n_ground = static_cast<int>((nnz - c.nnz_red - 1) / 2);  // its row and column went, one entry in both
+    c.ground_rows.reset(c.n_ground, "ground rows");
+    ground_rows_kernel<<<1, kWave, 0, s>>>(indptr.get(), indices.get(), c.ground, c.ground_rows.get());
     if (c.opts.keep_stiffness) {
         c.indptr = std::move(indptr);
         c.indices = std::move(indices);
@@ -465,6 +482,8 @@ void build_context(cn_context& c, const double* nodes_mm, std::int64_t n, const 
     op.off = {c.optr.get(), c.ocol.get(), c.oval.get(), nr, nr, c.nnz_red - nr};
     op.rowsum = c.rowsum.get();
     op.val64 = c.rval64.get();
+    op.ground_rows = c.ground_rows.get();
+    op.n_ground = c.n_ground;
     c.solver = std::make_unique<BlockSolver>(op, c.hier, s);
     c.ell_full_w = build_ell(c.reduced_view(), c.ell_full, s);
     if (!c.hier.levels.empty()) build_ell(c.hier.levels[0].scaled, c.ell_scaled, s);
@@ -776,6 +795,8 @@ std::unique_ptr<MatchedSolve> matched_solve(cn_context& c, const double* sigma_r
     op.off = {c.optr.get(), c.ocol.get(), ms->off32.get(), nr, nr, nnz_off};
     op.rowsum = ms->rs32.get();
     op.val64 = ms->v64.get();
+    op.ground_rows = c.ground_rows.get();
+    op.n_ground = c.n_ground;
     ms->solver = std::make_unique<BlockSolver>(op, ms->h, s);
     sync(s, "matched preconditioner");
     return ms;
@@ -814,6 +835,7 @@ void retry_missed(cn_context& c, cn::SolveStats& st, const cn::SolveOptions& opt
             auto ms = matched_solve(c, sigma + static_cast<std::int64_t>(col) * T);
             ++c.matched_preconditioners;
             r = ms->solver->solve(b1.get(), x1.get(), x0.get(), 1, opt);
+            sync(s, "matched solve");  // its buffers go with it
         } else {
             r = c.solver->solve(b1.get(), x1.get(), x0.get(), 1, opt);
         }
@@ -882,7 +904,6 @@ void uq_solve(cn_context& c, const double* sigma, int k, const cn_solve_options*
         sync(s, "uq initial guess");
         dx0 = c.d_x0.get();
     }
-    opt.take_constant = out != nullptr && out->v != nullptr;
     c.solver->set_multi(&u.mop);
     SolveStats st;
     try {

@@ -1460,76 +1460,91 @@ __global__ void __launch_bounds__(kWave) round_start_kernel(int k, double tolera
 // The constant part of a solution's error. The ground node takes whatever net current the residual has
 // left, so the whole potential is off by that over the ground's conductance, 4e-6 to 4e-5 of its norm
 // after a solve to 1e-6 where the rest of the error is 5e-7. With 1 the vector of ones,
-// x += 1 (1^T r) / (1^T A 1) takes it out (the A-norm projection of the error on 1; the residual changes
-// in the ground's own neighbours alone, by a twentieth of the tolerance; a column that it would take
-// above the tolerance, as a dipole all but touching a node can, keeps its solution). A is symmetric, so 1^T r is
-// sum_i (b_i - s_i x_i) with the row sums s = A 1, a pass over two vectors. (The recursive residual's sum
-// will not do: its FP32 rounding since the first iteration is what there is to take out.)
+// x += 1 (1^T r) / (1^T A 1) takes it out (the A-norm projection of the error on 1). A is symmetric and
+// its row sums s = A 1 vanish off the ground's neighbours, so 1^T r is the sum of b less that of s_i x_i
+// over those few rows: one pass over b, once a solve, and a kernel of a block per column after each
+// round. (The recursive residual's sum will not do: its FP32 rounding since the first iteration is what
+// there is to take out.) The residual changes in those rows alone, by a twentieth of the tolerance, and
+// its new norm follows from the old one; a column that it would take above the tolerance, as a dipole
+// all but touching a node can, keeps its solution. The shift goes into the copy handed out; the iterate
+// stays as solved.
+constexpr int kSumChunks = 8;
 
-// sums[block, c] = sum over the block's kWave rows of b - s x in FP64 (of s alone without b), a fixed
-// tree whatever K. s is (n), or (n, K) with SK.
-template <int K, bool SK>
+// sums[block, c] = FP64 sum over the block's kSumChunks * kWave rows of b, in an order that does not
+// depend on K.
+template <int K>
 __global__ void __launch_bounds__((kWave * K < 1024 ? kWave * K : 1024)) column_sum_kernel(
-    std::int64_t n, const float* __restrict__ b, const float* __restrict__ s, const double* __restrict__ x,
-    double* __restrict__ sums) {
-    __shared__ double tile[K][kWave + 1];
-    const std::int64_t r0 = static_cast<std::int64_t>(blockIdx.x) * kWave;
-    for (int t = threadIdx.x; t < kWave * K; t += blockDim.x) {
-        const std::int64_t row = r0 + t / K, at = row * K + t % K;
-        double v = 0.0;
-        if (row < n) {
-            const double sv = static_cast<double>(s[SK ? at : row]);
-            v = b != nullptr ? fma(-sv, x[at], static_cast<double>(b[at])) : sv;
-        }
-        tile[t % K][t / K] = v;
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1);
-    for (int c = threadIdx.x / kWave; c < K; c += blockDim.x / kWave) {
-        double v = tile[c][lane];
+    std::int64_t n, const float* __restrict__ b, double* __restrict__ sums) {
+    constexpr int WAVES = (kWave * K < 1024 ? kWave * K : 1024) / kWave, PER = K / WAVES;
+    __shared__ float tile[K][kWave + 1];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    double acc[PER] = {};
+    for (int q = 0; q < kSumChunks; ++q) {
+        const std::int64_t r0 = (static_cast<std::int64_t>(blockIdx.x) * kSumChunks + q) * kWave;
+        if (r0 >= n) break;  // whole blocks
+        for (int t = threadIdx.x; t < kWave * K; t += WAVES * kWave)
+            tile[t % K][t / K] = r0 + t / K < n ? b[r0 * K + t] : 0.0f;
+        __syncthreads();
 #pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + c] = v;
-    }
-}
-
-// out[c] = sum of the block sums of column c (one block per column, fixed order), over den[c * den_step]
-// when den is given (0 where that is not positive).
-__global__ void __launch_bounds__(kBlock) column_total_kernel(const double* __restrict__ sums, std::int64_t blocks,
-                                                              int K, const double* __restrict__ den, int den_step,
-                                                              double* __restrict__ out) {
-    __shared__ double s[kBlock];
-    const int c = blockIdx.x;
-    double acc = 0.0;
-    for (std::int64_t b = threadIdx.x; b < blocks; b += kBlock) acc += sums[b * K + c];
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+        for (int i = 0; i < PER; ++i) acc[i] += static_cast<double>(tile[wave + i * WAVES][lane]);
         __syncthreads();
     }
-    if (threadIdx.x != 0) return;
-    const double d = den != nullptr ? den[c * den_step] : 1.0;
-    out[c] = d > 0.0 ? s[0] / d : 0.0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        double v = acc[i];
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + wave + i * WAVES] = v;
+    }
 }
 
-// The shifts of the columns whose residual they took above the tolerance, to be undone; 0 elsewhere.
-__global__ void undo_shift_kernel(int K, double tolerance, const double* __restrict__ norms,
-                                  const double* __restrict__ bnorm, double* __restrict__ shift) {
-    const int c = threadIdx.x;
-    if (c < K) shift[c] = norms[c] > tolerance * bnorm[c] ? -shift[c] : 0.0;
+// Column c's shift (one block per column, fixed order) from b's block sums, the row sums s ((n), or (n, K)
+// with SK), x and r = b - A x; norms[c] becomes the norm of the residual with the shift.
+template <int K, bool SK>
+__global__ void __launch_bounds__(kBlock) constant_shift_kernel(
+    const double* __restrict__ sums, std::int64_t blocks, const std::int32_t* __restrict__ rows, int n_rows,
+    const float* __restrict__ s, const double* __restrict__ x, const double* __restrict__ r, double tolerance,
+    const double* __restrict__ bnorm, double* __restrict__ norms, double* __restrict__ shift) {
+    __shared__ double part[4][kBlock];
+    const int c = blockIdx.x, t = threadIdx.x;
+    double net = 0.0, ss = 0.0, s2 = 0.0, sr = 0.0;
+    for (std::int64_t b = t; b < blocks; b += kBlock) net += sums[b * K + c];
+    for (int i = t; i < n_rows; i += kBlock) {
+        const std::int64_t row = rows[i], at = row * K + c;
+        const double sv = static_cast<double>(s[SK ? at : row]);
+        net = fma(-sv, x[at], net);
+        ss += sv;
+        s2 = fma(sv, sv, s2);
+        sr = fma(sv, r[at], sr);
+    }
+    part[0][t] = net;
+    part[1][t] = ss;
+    part[2][t] = s2;
+    part[3][t] = sr;
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if (t < w)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) part[q][t] += part[q][t + w];
+        __syncthreads();
+    }
+    if (t != 0) return;
+    const double d = part[1][0] > 0.0 ? part[0][0] / part[1][0] : 0.0;
+    const double norm = sqrt(fmax(fma(d, fma(d, part[2][0], -2.0 * part[3][0]), norms[c] * norms[c]), 0.0));
+    const bool take = norm <= tolerance * bnorm[c];  // false where d is not finite
+    shift[c] = take ? d : 0.0;
+    if (take) norms[c] = norm;
 }
 
-// X = out = X + shift per column: the solution handed out, in place of a plain copy.
+// out = X + shift per column.
 template <int K>
-__global__ void shift_copy_kernel(std::int64_t count, const double* __restrict__ shift, double* __restrict__ X,
+__global__ void shift_copy_kernel(std::int64_t count, const double* __restrict__ shift, const double* __restrict__ X,
                                   double* __restrict__ out) {
     const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const double v = X[i] + shift[i % K];
-    X[i] = v;
-    out[i] = v;
+    if (i < count) out[i] = X[i] + shift[i % K];
 }
+
+std::int64_t sum_blocks(std::int64_t n) { return (n + kSumChunks * kWave - 1) / (kSumChunks * kWave); }
 
 std::int64_t gram_rows(std::int64_t n) { return (n + kGramBlocks - 1) / kGramBlocks; }
 
@@ -1866,8 +1881,8 @@ void BlockSolver::ensure(int K) {
     norms_.reset(K, "norms");
     bnorm_.reset(K, "right-hand-side norms");
     target_.reset(K, "targets");
-    shift_.reset(2 * static_cast<std::size_t>(K), "solution shifts");
-    col_sums_.reset(static_cast<std::size_t>((n() + kWave - 1) / kWave) * K, "column sums");
+    shift_.reset(K, "solution shifts");
+    col_sums_.reset(static_cast<std::size_t>(sum_blocks(n())) * K, "column sums");
     state_.reset(2 + 2 * kMaxBlock, "solver state");
     cap_k_ = K;
     drop_graphs();  // the captured iterations named the buffers just replaced
@@ -2091,8 +2106,17 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
                 zero);
         column_norms_kernel<K><<<1, kSmallThreads, 0, s_>>>(partials_.get(), kGramBlocks, norms);
     };
-    auto true_residual = [&](bool zero) {
-        residual_norms(zero, norms_.get());
+    // After a round: the residual's norms, with the shift of the columns that take it, and X.
+    auto round_residual = [&] {
+        residual_norms(false, norms_.get());
+        const auto shift = [&](auto sk, const float* rowsum) {
+            constant_shift_kernel<K, decltype(sk)::value><<<K, kBlock, 0, s_>>>(
+                col_sums_.get(), sum_blocks(nn), op_.ground_rows, op_.n_ground, rowsum, Xi, R64_.get(), opt.tolerance,
+                bnorm_.get(), norms_.get(), shift_.get());
+        };
+        multi_ ? shift(std::true_type{}, multi_->rowsum) : shift(std::false_type{}, op_.rowsum);
+        // Handed out before the wait: a further round writes it again.
+        shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift_.get(), Xi, X);
         d2h(rnorm.data(), norms_.get(), K, s_);
         sync(s_, "true residual");
     };
@@ -2100,6 +2124,8 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
         for (int c = 0; c < k; ++c) require(bnorm[c] > 0.0, "zero right-hand-side column " + std::to_string(c));
     };
     residual_norms(true, bnorm_.get());  // x_zero: R64 = B, so these are ||b_c||
+    constexpr int kSumThreads = kWave * K < 1024 ? kWave * K : 1024;
+    column_sum_kernel<K><<<static_cast<unsigned>(sum_blocks(nn)), kSumThreads, 0, s_>>>(nn, B, col_sums_.get());
     if (X0 != nullptr) {
         d2d(Xi, X0, static_cast<std::size_t>(nk), s_);
         residual_norms(false, norms_.get());
@@ -2121,7 +2147,6 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
     std::vector<int> host_state(2 + 2 * kMaxBlock, 0);
     bool use_graph = opt.use_graph;  // cleared for the rest of this solve if a capture fails
     int total_iters = 0;
-    bool handed_out = false;  // X holds the solution (written with the round's shift)
     std::vector<int> col_iters(K, 0);
     int slot = 0;
     while (kBlockWidths[slot] != K) ++slot;
@@ -2249,42 +2274,7 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
             sync(s_, "right-hand-side norms");
             check_bnorm();
         }
-        if (opt.take_constant) {  // the constant part of the error, and the solution handed out
-            const std::int64_t blocks = (nn + kWave - 1) / kWave;
-            constexpr int kSumThreads = kWave * K < 1024 ? kWave * K : 1024;
-            double* const shift = shift_.get();
-            const double* den = ground_g_.get();
-            const auto sum = [&](auto sk, const float* b, const float* rs) {
-                column_sum_kernel<K, decltype(sk)::value><<<static_cast<unsigned>(blocks), kSumThreads, 0, s_>>>(
-                    nn, b, rs, Xi, col_sums_.get());
-            };
-            if (multi_) {
-                sum(std::true_type{}, nullptr, multi_->rowsum);
-                column_total_kernel<<<K, kBlock, 0, s_>>>(col_sums_.get(), blocks, K, nullptr, 0, shift + K);
-                den = shift + K;
-                sum(std::true_type{}, B, multi_->rowsum);
-            } else {
-                if (!den) {  // once per solver: its operator does not change
-                    ground_g_.reset(1, "ground conductance");
-                    column_sum_kernel<1, false><<<static_cast<unsigned>(blocks), kWave, 0, s_>>>(
-                        nn, nullptr, op_.rowsum, nullptr, col_sums_.get());
-                    column_total_kernel<<<1, kBlock, 0, s_>>>(col_sums_.get(), blocks, 1, nullptr, 0, ground_g_.get());
-                    den = ground_g_.get();
-                }
-                sum(std::false_type{}, B, op_.rowsum);
-            }
-            column_total_kernel<<<K, kBlock, 0, s_>>>(col_sums_.get(), blocks, K, den, multi_ ? 1 : 0, shift);
-            shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift, Xi, X);
-            handed_out = true;
-        }
-        true_residual(false);
-        bool over = false;
-        for (int c = 0; c < k; ++c) over |= !(rnorm[c] <= opt.tolerance * bnorm[c]);
-        if (over && handed_out) {
-            undo_shift_kernel<<<1, kWave, 0, s_>>>(K, opt.tolerance, norms_.get(), bnorm_.get(), shift_.get());
-            shift_copy_kernel<K><<<grid_for(nk), kBlock, 0, s_>>>(nk, shift_.get(), Xi, X);
-            true_residual(false);
-        }
+        round_residual();
         double worst = 0.0;
         for (int c = 0; c < k; ++c) worst = std::max(worst, rnorm[c] / bnorm[c]);
         if (stats.refinements < kMaxRounds) {
@@ -2298,10 +2288,7 @@ SolveStats BlockSolver::solve_k(const float* B, double* X, const double* X0, int
         stats.column_iterations[c] = col_iters[c];
     }
     stats.iterations = total_iters;
-    if (!handed_out) {
-        d2d(X, Xi, static_cast<std::size_t>(nk), s_);
-        sync(s_, "solution copy");
-    }
+    if (stats.refinements == 0) d2d(X, Xi, static_cast<std::size_t>(nk), s_);
     return stats;
 }
 

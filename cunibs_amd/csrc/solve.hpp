@@ -64,10 +64,6 @@ struct SolveOptions {
     int check_every = 4;        // graph replays between host convergence reads
     bool use_graph = true;
     bool independent = false;   // k independent CG chains (diagonal Grams) instead of block CG
-    // Take the constant part out of the solution's error after each round. Only the potential sees it: a
-    // caller with a matrix per column that wants fields alone leaves it (0.25 ms of a 7.7 ms solve of 16
-    // conductivity draws, for the sums over every column's own row sums and the residual after them).
-    bool take_constant = true;
 };
 
 struct SolveStats {
@@ -86,11 +82,14 @@ struct SolveStats {
 //         y_i = sum_{j != i} a_ij (x_j - x_i) + s_i x_i, which keeps the FP32 product free of the
 //         cancellation between a stiffness row's entries (they sum to ~0)
 //   val64: FP64 values for the true residual
+//   ground_rows: the rows whose sums s_i are not zero but for rounding
 struct Operator {
     CsrView a32;
     CsrView off;
     const float* rowsum = nullptr;
     const double* val64 = nullptr;
+    const std::int32_t* ground_rows = nullptr;  // the rows with entries in the dropped ground column
+    int n_ground = 0;
 };
 
 constexpr int kMaxTissues = 16;
@@ -244,7 +243,7 @@ class BlockSolver {
     DeviceBuffer<double> partials_;  // kGramBlocks * 2 * K * K
     DeviceBuffer<double> red_;       // the partials summed over the blocks (2 K^2)
     DeviceBuffer<double> G_, TT_, AL_, D_, norms_, target_;  // AL_: kLag K x K coefficient slots
-    DeviceBuffer<double> shift_, col_sums_, ground_g_;  // the final constant shift of each column
+    DeviceBuffer<double> shift_, col_sums_;  // each column's constant shift; its right-hand side's block sums
     DeviceBuffer<double> bnorm_;  // ||b_c||, kept on the device for the first round's targets
     DeviceBuffer<float> g_x_[2], g_b_[2];  // the guess basis: FP32 solutions and their right-hand sides
     DeviceBuffer<double> g_mat_;           // its Grams, cross blocks and the last guess's coefficients

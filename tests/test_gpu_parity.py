@@ -167,6 +167,42 @@ def test_true_residual_in_fp64(single, gctx):
     assert r == pytest.approx(res.relative_residual, rel=1e-3, abs=1e-12)
 
 
+@pytest.mark.parametrize("k,own_sigma", [(1, False), (3, True), (8, False), (17, False)])
+def test_potentials_carry_no_constant_error(head8, coil, oracle_mod, k, own_sigma):
+    """The ground node takes the net current that a solve to 1e-6 leaves, which would shift the whole
+    potential by up to 4e-5 of its norm: what is handed out is off by less than the solve's own error,
+    and its residual is the one reported."""
+    import scipy.sparse as sp
+    from scipy.sparse.linalg import splu
+
+    from cunibs_amd import fem, synthetic
+    mesh = (head8.nodes_mm, head8.tet_nodes, head8.tet_tags, head8.skin_tris)
+    tables = [{2: 0.3 + 0.02 * i} for i in range(k)] if own_sigma else [{}]
+    ex = {"rhs": 1}
+    ctx = fem.SolverContext(*mesh)
+    try:
+        res = fem.solve_placements_block(ctx, coil.positions_m, coil.moments, synthetic.cap_sites(k, seed=31), 1e6,
+                                         potential=True, magnitude=False, metrics=False, extra=ex,
+                                         sigma=fem.conductivity_rows(tables) if own_sigma else None)
+        keep = np.arange(ctx.n_nodes) != ctx.ground_node
+    finally:
+        ctx.free()
+    for i, (r, b) in enumerate(zip(res, ex["rhs"])):
+        if i < len(tables):
+            own = fem.SolverContext(*mesh, conductivity={**fem.TISSUE_CONDUCTIVITY, **tables[i]})
+            rp, rc, rv = own.reduced()
+            own.free()
+            a = sp.csr_matrix((rv, rc, rp))
+            lu = splu(a.tocsc())
+        bb = b[keep].astype(np.float64)
+        want = lu.solve(bb)
+        err = r.v[keep] - want
+        assert abs(err.mean()) * np.sqrt(err.size) <= 1e-6 * np.linalg.norm(want)
+        residual = np.linalg.norm(bb - a @ r.v[keep]) / np.linalg.norm(bb)
+        # two FP64 evaluations of a residual 1e-6 of b, and FP32 row sums in the shift's part of its norm
+        assert residual == pytest.approx(r.relative_residual, rel=1e-5) and r.relative_residual <= 1e-6
+
+
 def test_gm_metrics_match_the_oracle_summary(single, gctx, oracle_mod):
     """metrics.py:209-243 on the GPU's own |E|: the device reduction equals the NumPy restatement."""
     from cunibs_amd import fem

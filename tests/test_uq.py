@@ -98,6 +98,24 @@ def test_placements_prepared_anew_keep_the_captured_iterations(head8, coil):
 
 
 @pytest.mark.gpu
+def test_asking_for_the_potential_changes_nothing_else(head8, coil):
+    from cunibs_amd import fem, synthetic, uq
+    ctx = fem.SolverContext(head8.nodes_mm, head8.tet_nodes, head8.tet_tags, head8.skin_tris)
+    try:
+        tags = ctx.uq_prepare(coil.positions_m, coil.moments, synthetic.SPHERE_SITE, 1e6)
+        sigma = uq.draw_lognormal(tags, 5, 0.2, seed=7)
+        plain = ctx.uq_solve(sigma, vectors=True)
+        asked = ctx.uq_solve(sigma, vectors=True, potential=True)
+    finally:
+        ctx.free()
+    for a, b in zip(plain, asked):
+        np.testing.assert_array_equal(a.E, b.E)
+        np.testing.assert_array_equal(a.magnE, b.magnE)
+        np.testing.assert_array_equal(a.metrics, b.metrics)
+        assert a.relative_residual == b.relative_residual
+
+
+@pytest.mark.gpu
 def test_per_placement_conductivities_match_fp64_solves(head4, coil, oracle_mod):
     """solve_placements_block(sigma=...): every placement of a block with its own conductivities,
     against the FP64 oracle built with that placement's table; the nominal row reproduces the
