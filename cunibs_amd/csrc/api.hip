@@ -194,7 +194,7 @@ struct cn_context {
     cn::MultiOperator blk_mop;
     struct Uq {
         bool ready = false;
-        cn::DeviceBuffer<float> rhs;                  // (T, n_red)
+        cn::DeviceBuffer<float> rhs, rhs_ground;      // (T, n_red), (T)
         cn::DeviceBuffer<float> dadt_nodes1;  // the placement's nodal dA/dt, one column
         // A draw block's operator values. They outlive uq_prepare (grow-only): captured iterations are
         // found again by these addresses, and a placement prepared anew met other ones more often than
@@ -673,6 +673,7 @@ void uq_initial_guess(cn_context& c) {
     c.stage_blk.put(dsig.get(), sig0.data(), T, s);
     c.d_B.ensure(nr * 1, "rhs block");
     combine_tissues(u.rhs.get(), nr, T, dsig.get(), 1, 1, c.d_B.get(), s);
+    balance_combined(c.d_B.get(), nr, 1, 1, u.rhs_ground.get(), T, dsig.get(), c.d_rhs_sums, s);
     c.d_X.ensure(nr * 1, "solution");
     SolveStats st = c.solver->solve(c.d_B.get(), c.d_X.get(), nullptr, 1, opt);
     u.nominal_iterations = st.iterations;
@@ -725,6 +726,7 @@ void uq_prepare(cn_context& c, const double* pos_m, const double* mom, std::int6
         u = std::move(next);
     }
     u.rhs.reset(static_cast<std::size_t>(T) * nr, "tissue rhs");
+    u.rhs_ground.reset(T, "tissue rhs");
     // The placement's dA/dt (one column), then the RHS of each tissue with unit conductivity.
     std::vector<double> tf(16);
     std::vector<std::int32_t> degen(1);
@@ -740,8 +742,8 @@ void uq_prepare(cn_context& c, const double* pos_m, const double* mom, std::int6
         tissue_neg_vc(c.vols32.get(), c.tags.get(), m, present[t], negvc.get(), s);
         element_pass(u.dadt_nodes1.get(), c.tets.get(), c.g32.get(), negvc.get(), m, 1, 1, nullptr, q.get(),
                      c.corner_pos.get(), s);
-        node_rhs(q.get(), c.n2c_ptr.get(), n, 1, 1, c.ground, u.rhs.get() + static_cast<std::int64_t>(t) * nr, nullptr,
-                 c.d_rhs_sums, s);
+        tissue_rhs(q.get(), c.n2c_ptr.get(), n, c.ground, u.rhs.get() + static_cast<std::int64_t>(t) * nr,
+                   u.rhs_ground.get() + t, s);
     }
     u.sum.reset(m, "|E| sum");
     u.sumsq.reset(m, "|E| sum of squares");
@@ -869,6 +871,7 @@ void uq_solve(cn_context& c, const double* sigma, int k, const cn_solve_options*
     combine_tissues(c.tissue.off.get(), nnz_off, T, u.sigma.get(), k, K, u.off_k.get(), s);
     combine_tissues(c.tissue.rowsum.get(), nr, T, u.sigma.get(), k, K, u.rowsum_k.get(), s);
     combine_tissues(u.rhs.get(), nr, T, u.sigma.get(), k, K, c.d_B.get(), s);
+    balance_combined(c.d_B.get(), nr, k, K, u.rhs_ground.get(), T, u.sigma.get(), c.d_rhs_sums, s);
     u.mop.width = K;
     u.mop.off_vals = u.off_k.get();
     u.mop.rowsum = u.rowsum_k.get();

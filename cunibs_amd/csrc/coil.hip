@@ -289,9 +289,20 @@ __global__ void element_pass_kernel(const float* __restrict__ nodal, const std::
 // block takes kRhsRows nodes and writes their columns' FP64 sums (fixed tree) to sums (blocks, K).
 constexpr int kRhsRows = kWave;
 
+// sums[block, c] = the FP64 sum of a block's kRhsRows rows of column c, a butterfly per column.
+__device__ __forceinline__ void block_sums(const float (*tile)[kRhsRows + 1], int K, double* __restrict__ sums) {
+    const int lane = threadIdx.x & (kWave - 1), waves = blockDim.x / kWave;
+    for (int c = threadIdx.x / kWave; c < K; c += waves) {
+        double v = static_cast<double>(tile[c][lane]);
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + c] = v;
+    }
+}
+
 __global__ void node_rhs_kernel(const float* __restrict__ q, const std::int32_t* __restrict__ ptr, std::int64_t n,
                                 int k, int K, int ground, float* __restrict__ B, float* __restrict__ b_full,
-                                double* __restrict__ sums) {
+                                float* __restrict__ b_ground, double* __restrict__ sums) {
     __shared__ float tile[32][kRhsRows + 1];  // K <= 32
     const std::int64_t n0 = static_cast<std::int64_t>(blockIdx.x) * kRhsRows;
     for (int t = threadIdx.x; t < kRhsRows * K; t += blockDim.x) {
@@ -301,18 +312,39 @@ __global__ void node_rhs_kernel(const float* __restrict__ q, const std::int32_t*
         if (node < n) {
             for (int p = ptr[node]; p < ptr[node + 1]; ++p) acc += q[static_cast<std::int64_t>(p) * K + c];
             if (b_full != nullptr && c < k) b_full[c * n + node] = acc;
-            if (node != ground) B[(node - (node > ground)) * K + c] = acc;
+            if (node != ground)
+                B[(node - (node > ground)) * K + c] = acc;
+            else if (b_ground != nullptr)
+                b_ground[c] = acc;
         }
         tile[c][t / K] = acc;
     }
     __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1), waves = blockDim.x / kWave;
-    for (int c = threadIdx.x / kWave; c < K; c += waves) {
-        double v = static_cast<double>(tile[c][lane]);
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-        if (lane == 0) sums[static_cast<std::int64_t>(blockIdx.x) * K + c] = v;
+    if (sums != nullptr) block_sums(tile, K, sums);
+}
+
+// The same sums of right-hand sides that were combined from the tissues' (nr, K), with the ground node's
+// entry of each (the sum of its tissues' by the column's conductivities) as a last row.
+__global__ void combined_sums_kernel(const float* __restrict__ B, std::int64_t nr, int k, int K,
+                                     const float* __restrict__ b_ground, int T, const double* __restrict__ sigma,
+                                     double* __restrict__ sums) {
+    __shared__ float tile[32][kRhsRows + 1];  // K <= 32
+    const std::int64_t r0 = static_cast<std::int64_t>(blockIdx.x) * kRhsRows;
+    for (int t = threadIdx.x; t < kRhsRows * K; t += blockDim.x) {
+        const std::int64_t row = r0 + t / K;
+        const int c = t % K;
+        float v = 0.f;
+        if (row < nr) {
+            v = B[row * K + c];
+        } else if (row == nr && c < k) {
+            double acc = 0.0;
+            for (int q = 0; q < T; ++q) acc = fma(sigma[c * T + q], static_cast<double>(b_ground[q]), acc);
+            v = static_cast<float>(acc);
+        }
+        tile[c][t / K] = v;
     }
+    __syncthreads();
+    block_sums(tile, K, sums);
 }
 
 // The right-hand side of a field without sources sums to zero over all nodes; its FP32 rounding
@@ -404,10 +436,26 @@ void node_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int k, in
     const std::int64_t blocks = (n + kRhsRows - 1) / kRhsRows;
     if (blocks <= 0) return;
     sums.ensure(static_cast<std::size_t>(blocks) * K, "right-hand-side sums");
-    node_rhs_kernel<<<static_cast<unsigned>(blocks), std::min(kRhsRows * K, 1024), 0, s>>>(q, ptr, n, k, K, ground, B,
-                                                                                          b_full, sums.get());
+    node_rhs_kernel<<<static_cast<unsigned>(blocks), std::min(kRhsRows * K, 1024), 0, s>>>(
+        q, ptr, n, k, K, ground, B, b_full, nullptr, sums.get());
     if (n > 1 && k > 0)
         balance_rhs_kernel<<<static_cast<unsigned>(k), kBlock, 0, s>>>(sums.get(), blocks, n, K, ground, B, b_full);
+}
+
+void tissue_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int ground, float* b, float* b_ground,
+                hipStream_t s) {
+    if (const unsigned blocks = grid_for(n, kRhsRows))
+        node_rhs_kernel<<<blocks, kRhsRows, 0, s>>>(q, ptr, n, 1, 1, ground, b, nullptr, b_ground, nullptr);
+}
+
+void balance_combined(float* B, std::int64_t nr, int k, int K, const float* b_ground, int T, const double* sigma,
+                      DeviceBuffer<double>& sums, hipStream_t s) {
+    if (nr <= 0 || k <= 0) return;
+    const std::int64_t blocks = (nr + 1 + kRhsRows - 1) / kRhsRows;
+    sums.ensure(static_cast<std::size_t>(blocks) * K, "right-hand-side sums");
+    combined_sums_kernel<<<static_cast<unsigned>(blocks), std::min(kRhsRows * K, 1024), 0, s>>>(B, nr, k, K, b_ground, T,
+                                                                                               sigma, sums.get());
+    balance_rhs_kernel<<<static_cast<unsigned>(k), kBlock, 0, s>>>(sums.get(), blocks, nr + 1, K, 0, B, nullptr);
 }
 
 }  // namespace cn

@@ -29,6 +29,13 @@ void corner_positions(const std::int32_t* idx, std::int64_t count, std::int32_t*
 // each column brought to a zero sum over all nodes; `sums` is scratch (grow-only).
 void node_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int k, int K, int ground, float* B,
               float* b_full, DeviceBuffer<double>& sums, hipStream_t s);
+// The same of one column, as gathered, and the ground node's entry; and the columns of a block combined
+// from T such vectors by sigma (K x T) brought to a zero sum with theirs (b_ground: T). Combining rounds
+// every entry anew, so what the vectors' own sums were does not matter.
+void tissue_rhs(const float* q, const std::int32_t* ptr, std::int64_t n, int ground, float* b, float* b_ground,
+                hipStream_t s);
+void balance_combined(float* B, std::int64_t nr, int k, int K, const float* b_ground, int T, const double* sigma,
+                      DeviceBuffer<double>& sums, hipStream_t s);
 
 // post.hip
 void scatter_potential(const double* X, std::int64_t n, int k, int K, int ground, double* v, hipStream_t s);

@@ -116,6 +116,27 @@ def test_asking_for_the_potential_changes_nothing_else(head8, coil):
 
 
 @pytest.mark.gpu
+def test_draws_carry_no_net_current(head8, coil):
+    """A draw's right-hand side is brought to a zero sum after its tissues' vectors are combined, so its
+    potential is off by no more of a constant than a block's of the same conductivities (1e-6 of its norm
+    each; up to 7e-6 if the tissues' vectors are balanced instead, whose combination rounds anew)."""
+    from cunibs_amd import fem, synthetic, uq
+    ctx = fem.SolverContext(head8.nodes_mm, head8.tet_nodes, head8.tet_tags, head8.skin_tris)
+    try:
+        for site in synthetic.cap_sites(4, seed=31):
+            tags = ctx.uq_prepare(coil.positions_m, coil.moments, site, 1e6)
+            sigma = uq.draw_lognormal(tags, 3, 0.2, seed=2)
+            got = ctx.uq_solve(sigma, potential=True)
+            rows = fem.conductivity_rows([dict(zip(tags, map(float, r))) for r in sigma])
+            want = fem.solve_placements_block(ctx, coil.positions_m, coil.moments, [site] * 3, 1e6, potential=True,
+                                              sigma=rows)
+            for a, b in zip(got, want):
+                assert abs((a.v - b.v).mean()) * np.sqrt(a.v.size) <= 2e-6 * np.linalg.norm(b.v)
+    finally:
+        ctx.free()
+
+
+@pytest.mark.gpu
 def test_per_placement_conductivities_match_fp64_solves(head4, coil, oracle_mod):
     """solve_placements_block(sigma=...): every placement of a block with its own conductivities,
     against the FP64 oracle built with that placement's table; the nominal row reproduces the
