@@ -1508,6 +1508,7 @@ __global__ void __launch_bounds__(kBlock) constant_shift_kernel(
     __shared__ double part[4][kBlock];
     const int c = blockIdx.x, t = threadIdx.x;
     double net = 0.0, ss = 0.0, s2 = 0.0, sr = 0.0;
+#pragma unroll 8
     for (std::int64_t b = t; b < blocks; b += kBlock) net += sums[b * K + c];
     for (int i = t; i < n_rows; i += kBlock) {
         const std::int64_t row = rows[i], at = row * K + c;
