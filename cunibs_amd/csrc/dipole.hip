@@ -59,9 +59,10 @@ constexpr int kNarrow = 4;  // placements up to which a block of the box passes 
 constexpr std::int64_t kSplitTasks8 = 2048;
 constexpr std::int64_t kSplitTasks4 = 8192;
 
-// LDS added to a workgroup that runs beside a solve: one box or node workgroup a CU then leaves the
-// solve's kernels their wave slots (a 16-wide sweep at 330,000 nodes: 35.2 ms with the CUs filled,
-// 33.9 ms so; 97.6 and 96.5 at a million).
+// LDS added to a workgroup that runs beside a solve, so that it leaves the solve's kernels their wave
+// slots: of 160 KB a CU holds one workgroup of the box passes or of node_split_kernel with shared waves,
+// two of the other node passes (16-wide sweeps: at 213,000 nodes 25.6 ms with the CUs filled, 24.8 so; at
+// 966,000 nodes 97.3 and 96.4; a general coil's at 95,000 nodes 28.3 and 25.2).
 constexpr std::size_t kBesideLds = 60 * 1024;
 
 // tables layout (floats): points of order 8, points of order 6, then for child order 8 and 6 the
@@ -688,30 +689,38 @@ __global__ void __launch_bounds__(kDipoleThreads) node_split_kernel(NodeArgs a) 
     }
 }
 
-// Every node of a mesh without boxes, for a coil whose moments differ in direction: one node a lane, so
-// that small meshes fill the machine (eight nodes a thread, the shape of the raw entry point's kernel,
-// took 383 us for 89,000 nodes and 1,500 dipoles).
-__global__ void __launch_bounds__(kBlock) node_given_kernel(NodeArgs a) {
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) + wave;
-    if (t >= static_cast<std::int64_t>(a.n_chunks) * a.K) return;  // whole wavefronts
-    const int c = static_cast<int>(t % a.K);
-    const std::int64_t i = t / a.K * kWave + lane;
-    const std::int64_t node = min(i, a.n - 1);
-    float o[3] = {0.f, 0.f, 0.f};
-    if (c < a.k) {
-        const float r[3] = {static_cast<float>(a.nodes_mm[3 * node] * 1e-3 - a.origin[3 * c]),
-                            static_cast<float>(a.nodes_mm[3 * node + 1] * 1e-3 - a.origin[3 * c + 1]),
-                            static_cast<float>(a.nodes_mm[3 * node + 2] * 1e-3 - a.origin[3 * c + 2])};
-        float v[3];
-        given_sum(a, c, r, v);
-        turn<false>(a, c, v[0], v[1], v[2], o);
-    }
-    if (i >= a.n) return;
+// Placement c's sum in the caller's order at this lane's node, written there.
+__device__ __forceinline__ void write_given(const NodeArgs& a, int c, std::int64_t node, bool mine) {
+    const float r[3] = {static_cast<float>(a.nodes_mm[3 * node] * 1e-3 - a.origin[3 * c]),
+                        static_cast<float>(a.nodes_mm[3 * node + 1] * 1e-3 - a.origin[3 * c + 1]),
+                        static_cast<float>(a.nodes_mm[3 * node + 2] * 1e-3 - a.origin[3 * c + 2])};
+    float v[3], o[3];
+    given_sum(a, c, r, v);
+    turn<false>(a, c, v[0], v[1], v[2], o);
+    if (!mine) return;
     float* p = a.out + node * 3 * a.K + c;
     p[0] = o[0];
     p[a.K] = o[1];
     p[2 * a.K] = o[2];
+}
+
+// Every node of a mesh without boxes, for a coil whose moments differ in direction: one node a lane, so
+// that small meshes fill the machine (eight nodes a thread, the shape of the raw entry point's kernel,
+// took 383 us for 89,000 nodes and 1,500 dipoles). A capped grid walks the nodes.
+__global__ void __launch_bounds__(kBlock) node_given_kernel(NodeArgs a) {
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const std::int64_t tasks = static_cast<std::int64_t>(a.n_chunks) * a.K;
+    for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) + wave; t < tasks;
+         t += static_cast<std::int64_t>(gridDim.x) * (kBlock / kWave)) {
+        const int c = static_cast<int>(t % a.K);
+        const std::int64_t i = t / a.K * kWave + lane, node = min(i, a.n - 1);
+        if (c < a.k) {
+            write_given(a, c, node, i < a.n);
+        } else if (i < a.n) {
+            float* p = a.out + node * 3 * a.K + c;
+            p[0] = p[a.K] = p[2 * a.K] = 0.f;
+        }
+    }
 }
 
 double cheb_point(int i, int p) { return std::cos((i + 0.5) * M_PI / p); }
@@ -1004,7 +1013,7 @@ void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int
     };
     const std::int64_t tasks = static_cast<std::int64_t>(a.n_chunks) * K;
     if (!d.parallel && !d.boxes) {
-        node_given_kernel<<<grid_for(tasks, kBlock / kWave), kBlock, 0, s>>>(a);
+        node_given_kernel<<<capped((tasks + kBlock / kWave - 1) / (kBlock / kWave)), kBlock, pad, s>>>(a);
     } else if (k > 8 && a.n_chunks >= kWideMinChunks) {
         const std::size_t lds = std::max(sizeof(float) * static_cast<std::size_t>(kWave) * (3 * K + 1), pad);
         const unsigned grid = capped(a.n_chunks);

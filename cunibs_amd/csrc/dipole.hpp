@@ -54,8 +54,9 @@ void set_coil(DipoleSet& d, const BoxTree& t, const double* pos_m, const double*
               std::int64_t n_dip, hipStream_t s);
 
 // out (n, 3, K) = scale sum_j m_j x (r - s_j) / |r - s_j|^3 for the k placements with coil frames tf
-// (k x 16, host; columns past k are zero). max_blocks > 0 caps the grid of the last pass; `beside` keeps
-// the footprint small next to a solve on another stream.
+// (k x 16, host; columns past k are zero). max_blocks > 0 caps the grid of the passes over the nodes (not
+// that of the box passes before them); `beside` keeps the footprint small next to a solve on another
+// stream.
 void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int64_t n, const double* tf, int k, int K,
                 float scale, float* out, int max_blocks, bool beside, hipStream_t s);
 

@@ -88,7 +88,9 @@ typedef struct {
                            level (0 = chosen from each level's shape) */
     int32_t coil_blocks; /* cn_solve_sweep: workgroups of the next block's dA/dt while it overlaps
                             the current block's solve (0 = the full grid); fewer leave the solve
-                            more of the device */
+                            more of the device. On meshes of 100,000 nodes and more the passes over
+                            clusters of the mesh come first, on their full grid; the cap holds for
+                            the passes over the nodes */
     int32_t layout;     /* finest level's operator in the row kernels: 0 = the sliced ELL copy
                            (built when every row has at most 24 entries) for blocks of up to 4
                            columns and CSR above, 1 = CSR, 2 = the ELL copy at every width; the
@@ -199,7 +201,8 @@ typedef struct {
     double* relative_residual; /* (k) final FP64 true residual / ||b|| */
     float* dadt_elm;           /* (k, n_tets, 3) element dA/dt */
     float* dadt_nodes;         /* (k, n_nodes, 3) nodal dA/dt */
-    float* rhs;                /* (k, n_nodes) right-hand side before grounding */
+    float* rhs;                /* (k, n_nodes) right-hand side before grounding, as the solve takes it: each
+                                  column's rounding is balanced, so that it sums to zero */
     int32_t* degenerate;       /* (k) 1 where the handle left the frame undefined */
     float* E_slots;            /* (k, n_slots, 3) recovered field on its slots (recovery != raw) */
     double* x0;                /* (k, n_reduced) the initial guess PCG started from (zeros if cold) */

@@ -82,3 +82,30 @@ def test_right_hand_sides_sum_to_zero(ctx, k):
                                magnitude=False, metrics=False, extra=ex, tolerance=0.5)
     b = ex["rhs"].astype(np.float64)
     assert np.all(np.abs(b.sum(1)) <= 2.0 * 2.0**-24 * np.abs(b).max(1))
+
+
+def bent_coil(dipoles, tilt_deg=14.0):
+    """Two wings tilted towards the head, whose moments differ in direction."""
+    coil = synthetic.figure8_coil(seed=3, per_layer=-(-dipoles // 6))
+    pos, mom = coil.positions_m[:dipoles].copy(), coil.moments[:dipoles].copy()
+    for side in (-1.0, 1.0):
+        t, wing = side * np.radians(tilt_deg), pos[:, 0] * side > 0
+        turn = np.array([[np.cos(t), 0.0, -np.sin(t)], [0.0, 1.0, 0.0], [np.sin(t), 0.0, np.cos(t)]])
+        pos[wing], mom[wing] = pos[wing] @ turn.T, mom[wing] @ turn.T
+    return pos, mom
+
+
+def test_a_general_coils_sweep_equals_its_blocks(ctx):
+    """The N-body beside a solve, on a capped grid, for a coil whose moments differ."""
+    from cunibs_amd import fem
+    pos, mom = bent_coil(900)
+    sites = synthetic.cap_sites(11, seed=9, distance_range_mm=(12.0, 14.0))
+    blocks = [r.metrics for i in range(0, 11, 4)
+              for r in fem.solve_placements_block(ctx, pos, mom, sites[i:i + 4], 1e6, magnitude=False)]
+    try:
+        for cap in (0, 1, 7, 100):
+            ctx.set_tuning(coil_blocks=cap)
+            sweep = fem.solve_sweep(ctx, pos, mom, sites, 1e6, block_k=4, recycle=0)
+            np.testing.assert_array_equal(sweep["metrics"], np.stack(blocks))
+    finally:
+        ctx.set_tuning(coil_blocks=0)
