@@ -52,18 +52,31 @@ constexpr std::int64_t kBoxMinDipoles = 256;
 constexpr std::int64_t kBoxDeepNodes = 400000;
 constexpr std::int64_t kBoxDeeperNodes = 3200000;
 
-// Chunks from which a wide block's node pass fills the machine with a block per chunk, and (chunk,
-// placement) tasks below which eight and four waves share one.
+// Chunks from which a wide block's node pass takes a block per chunk (at 412,000 nodes, 6,600 chunks: 16
+// and 32 placements of 1,800 dipoles 1357 and 2655 us so, 1333 and 2508 with waves sharing a chunk), and
+// (chunk, placement) tasks below which eight and four waves share one (one placement at 7,400 nodes has
+// 116 tasks: 15 us for 964 dipoles).
 constexpr int kWideMinChunks = 8192;
 constexpr int kNarrow = 4;  // placements up to which a block of the box passes takes two points a lane
 constexpr std::int64_t kSplitTasks8 = 2048;
 constexpr std::int64_t kSplitTasks4 = 8192;
 
+// (chunk, placement) tasks from which near chunks go on a list: 4 placements of 4,000 dipoles at 213,000
+// nodes (18,000 tasks) 1175 us without and 1204 with it, 16 (72,000) 3604 and 3102; 16 at 125,000 (39,000)
+// 2712 and 2594; 4 at 667,000 (41,000) 1938 and 1728.
+constexpr std::int64_t kListTasks = 32768;
+static_assert(kListTasks <= 9 * kWideMinChunks, "node_wide_kernel leaves near chunks to the list");
+
 // LDS added to a workgroup that runs beside a solve, so that it leaves the solve's kernels their wave
 // slots: of 160 KB a CU holds one workgroup of the box passes or of node_split_kernel with shared waves,
 // two of the other node passes (16-wide sweeps: at 213,000 nodes 25.6 ms with the CUs filled, 24.8 so; at
-// 966,000 nodes 97.3 and 96.4; a general coil's at 95,000 nodes 28.3 and 25.2).
+// 966,000 nodes 97.3 and 96.4; a general coil's at 95,000 nodes 28.3 and 25.2). The box and node passes
+// of many dipoles whose moments differ take longer than the solves beside them, and then take more of
+// the machine (32-wide sweeps at 138,000 nodes: 4,000 dipoles 32.3 ms with the wide pad, 28.4 so, 2,600
+// 26.3 and 24.9, 1,800 22.6 and 22.8).
 constexpr std::size_t kBesideLds = 60 * 1024;
+constexpr std::size_t kBesideHeavyLds = 24 * 1024;
+constexpr int kHeavyDipoles = 2304;
 
 // tables layout (floats): points of order 8, points of order 6, then for child order 8 and 6 the
 // matrices T[half][child point][parent point] (parent order 8).
@@ -385,6 +398,7 @@ struct NodeArgs {
     int k, K;
     float scale;
     float* out;
+    const unsigned char* near_flag;  // (n_chunks, k): the chunks on the list
 };
 
 struct Chunk {
@@ -399,12 +413,8 @@ __device__ __forceinline__ Chunk chunk_at(const NodeArgs& a, int chunk) {
     return {n0, static_cast<int>(min(static_cast<std::int64_t>(kWave), a.n - n0)), -1, chunk};
 }
 
-// Whether placement c at this chunk takes every dipole in the caller's order: some cluster (lane q
-// testing cluster q) within kCloseMm of it.
-template <bool PAR>
-__device__ __forceinline__ bool takes_given(const NodeArgs& a, const Chunk& ch, int c) {
-    if constexpr (PAR) return false;
-    if (ch.leaf < 0) return true;
+// Whether some cluster (lane q testing cluster q) of placement c lies within kCloseMm of this chunk.
+__device__ __forceinline__ bool close_by(const NodeArgs& a, const Chunk& ch, int c) {
     const double* f = a.frames + 16 * c;
     const double* sp = a.spheres + 4 * (threadIdx.x & (kWave - 1));
     const double* ball = a.ball + 4 * static_cast<std::int64_t>(ch.id);
@@ -415,6 +425,18 @@ __device__ __forceinline__ bool takes_given(const NodeArgs& a, const Chunk& ch, 
         d2 += d * d;
     }
     return __ballot(sqrt(d2) - sp[3] < (kCloseMm + ball[3]) * 1e-3) != 0;
+}
+
+// How a node pass treats the chunks near a coil: a planar coil's like any other; else it sums every dipole
+// there in the caller's order itself, or leaves that to near_given_kernel (as near_chunks_kernel has found;
+// the pass keeps its registers for the rest).
+enum class Near { kPlain, kSum, kListed };
+
+template <Near NEAR>
+__device__ __forceinline__ bool takes_given(const NodeArgs& a, const Chunk& ch, int c) {
+    if constexpr (NEAR == Near::kListed) return a.near_flag[static_cast<std::int64_t>(ch.id) * a.k + c] != 0;
+    if constexpr (NEAR == Near::kSum) return close_by(a, ch, c);
+    return false;
 }
 
 struct Weights {
@@ -545,9 +567,11 @@ __device__ __forceinline__ void turn(const NodeArgs& a, int c, float ax, float a
 // The nodes of wide blocks on large meshes: one chunk per block and pass, a wave taking every eighth
 // placement. The chunk's (64, 3, K) outputs are gathered in LDS and written as one contiguous run (a
 // wave's own three stores touch 64 lines of 12 K bytes each; eight placements a block measured 15 %
-// slower). Bound by the latency of the values' scalar loads.
+// slower). Bound by the latency of the values' scalar loads. Chunks taken in the caller's order are left
+// to near_given_kernel.
 template <bool PAR>
 __global__ void __launch_bounds__(kDipoleThreads) __attribute__((amdgpu_waves_per_eu(6))) node_wide_kernel(NodeArgs a) {
+    constexpr Near NEAR = PAR ? Near::kPlain : Near::kListed;
     extern __shared__ float lds[];  // (64, 3 K + 1)
     const int K = a.K, k = a.k, ld = 3 * K + 1;
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -560,19 +584,13 @@ __global__ void __launch_bounds__(kDipoleThreads) __attribute__((amdgpu_waves_pe
         for (int c = wave; c < K; c += kSlices) {
             float o[3] = {0.f, 0.f, 0.f};
             if (c < k) {
-                const bool given = takes_given<PAR>(a, ch, c);
+                const bool given = takes_given<NEAR>(a, ch, c);
                 const unsigned long long cum = ch.leaf >= 0 ? a.far[static_cast<std::int64_t>(ch.leaf) * k + c] : 0ull;
                 const float r[3] = {static_cast<float>(x[0] * 1e-3 - a.origin[3 * c]),
                                     static_cast<float>(x[1] * 1e-3 - a.origin[3 * c + 1]),
                                     static_cast<float>(x[2] * 1e-3 - a.origin[3 * c + 2])};
                 float ax = 0.f, ay = 0.f, az = 0.f;
-                if (given) {
-                    float v[3];
-                    given_sum(a, c, r, v);
-                    ax = v[0];
-                    ay = v[1];
-                    az = v[2];
-                } else if (cum != 0) {
+                if (!given && cum != 0) {
                     const UniformFloats v =
                         uniform(a.values + (static_cast<std::int64_t>(ch.leaf - a.leaf_first) * k + c) * kLeafValues);
                     float bx, by, bz;
@@ -609,8 +627,9 @@ __global__ void __launch_bounds__(kDipoleThreads) __attribute__((amdgpu_waves_pe
 // The nodes of narrow blocks, and of meshes with few chunks: WP waves share one chunk of one placement
 // (a slice each of the near dipoles, the first two half of the interpolation), so that a single
 // placement still fills the machine.
-template <bool PAR, int WP>
+template <Near NEAR, int WP>
 __global__ void __launch_bounds__(kDipoleThreads) node_split_kernel(NodeArgs a) {
+    constexpr bool PAR = NEAR == Near::kPlain;
     static_assert(WP >= 2, "the interpolation is shared by two waves");
     constexpr int GROUPS = kSlices / WP, PER = kSlices / WP;
     __shared__ float part[GROUPS][kSlices + 2][3][kWave];
@@ -627,18 +646,20 @@ __global__ void __launch_bounds__(kDipoleThreads) node_split_kernel(NodeArgs a) 
         unsigned long long cum = 0;
         bool given = false;
         if (c < k) {
-            given = takes_given<PAR>(a, ch, c);
+            given = takes_given<NEAR>(a, ch, c);
             cum = ch.leaf >= 0 ? a.far[static_cast<std::int64_t>(ch.leaf) * k + c] : 0ull;
             const double x[3] = {a.nodes_mm[3 * node], a.nodes_mm[3 * node + 1], a.nodes_mm[3 * node + 2]};
             const float r[3] = {static_cast<float>(x[0] * 1e-3 - a.origin[3 * c]),
                                 static_cast<float>(x[1] * 1e-3 - a.origin[3 * c + 1]),
                                 static_cast<float>(x[2] * 1e-3 - a.origin[3 * c + 2])};
             if (given) {
-                if (q == 0) {
-                    float v[3];
-                    given_sum(a, c, r, v);
+                if constexpr (NEAR == Near::kSum) {
+                    if (q == 0) {
+                        float v[3];
+                        given_sum(a, c, r, v);
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) part[g][0][d][lane] = v[d];
+                        for (int d = 0; d < 3; ++d) part[g][0][d][lane] = v[d];
+                    }
                 }
             } else if (q < 2) {
                 float ax = 0.f, ay = 0.f, az = 0.f;
@@ -668,7 +689,7 @@ __global__ void __launch_bounds__(kDipoleThreads) node_split_kernel(NodeArgs a) 
             }
         }
         __syncthreads();
-        if (q == 0 && t0 + g < tasks && lane < ch.cnt) {
+        if (q == 0 && t0 + g < tasks && lane < ch.cnt && !(NEAR == Near::kListed && given)) {
             float o[3] = {0.f, 0.f, 0.f};
             if (c < k) {
                 float v[3];
@@ -720,6 +741,34 @@ __global__ void __launch_bounds__(kBlock) node_given_kernel(NodeArgs a) {
             float* p = a.out + node * 3 * a.K + c;
             p[0] = p[a.K] = p[2 * a.K] = 0.f;
         }
+    }
+}
+
+// flag[chunk, c]: whether placement c takes the chunk in the caller's order; near[c] = those chunks, in no
+// order. One wavefront per (chunk, placement). `count` starts at zero.
+__global__ void __launch_bounds__(kBlock) near_chunks_kernel(NodeArgs a, unsigned char* __restrict__ flag,
+                                                             std::int32_t* __restrict__ near,
+                                                             std::int32_t* __restrict__ count) {
+    const std::int64_t w = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
+    if (w >= static_cast<std::int64_t>(a.n_chunks) * a.k) return;  // whole wavefronts
+    const int chunk = static_cast<int>(w / a.k), c = static_cast<int>(w % a.k);
+    const bool given = close_by(a, chunk_at(a, chunk), c);
+    if ((threadIdx.x & (kWave - 1)) != 0) return;
+    flag[w] = given;
+    if (given) near[static_cast<std::int64_t>(c) * a.n_chunks + atomicAdd(count + c, 1)] = chunk;
+}
+
+// Placement blockIdx.y at its near chunks, one a wavefront: in the node passes of a wide block the waves
+// that share a chunk, or a block, would wait for the one that sums every dipole (32 placements of 4,000
+// dipoles at 125,000 nodes: 5.0 to 4.5 ms; with two chunks a wavefront 4.9, with four 5.5).
+__global__ void __launch_bounds__(kBlock) near_given_kernel(NodeArgs a, const std::int32_t* __restrict__ near,
+                                                            const std::int32_t* __restrict__ count) {
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = blockIdx.y, chunks = count[c];
+    for (int q = static_cast<int>(blockIdx.x) * (kBlock / kWave) + wave; q < chunks;
+         q += static_cast<int>(gridDim.x) * (kBlock / kWave)) {
+        const Chunk ch = chunk_at(a, near[static_cast<std::int64_t>(c) * a.n_chunks + q]);
+        write_given(a, c, ch.n0 + min(lane, ch.cnt - 1), lane < ch.cnt);
     }
 }
 
@@ -940,7 +989,7 @@ void set_coil(DipoleSet& d, const BoxTree& t, const double* pos_m, const double*
 void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int64_t n, const double* tf, int k, int K,
                 float scale, float* out, int max_blocks, bool beside, hipStream_t s) {
     if (n <= 0 || k <= 0) return;
-    const std::size_t pad = beside ? kBesideLds : 0;
+    const std::size_t pad = !beside ? 0 : d.boxes && !d.parallel && d.n >= kHeavyDipoles ? kBesideHeavyLds : kBesideLds;
     require(d.n >= 1, "no coil has been set");
     d.frames.ensure(16 * static_cast<std::size_t>(k), "coil frames");
     d.origin.ensure(3 * static_cast<std::size_t>(k), "coil origins");
@@ -1012,6 +1061,18 @@ void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int
         return static_cast<unsigned>(max_blocks > 0 ? std::min<std::int64_t>(grid, max_blocks) : grid);
     };
     const std::int64_t tasks = static_cast<std::int64_t>(a.n_chunks) * K;
+    // Wide blocks of a coil whose moments differ: the near chunks on a list.
+    const bool listed = !d.parallel && d.boxes && static_cast<std::int64_t>(a.n_chunks) * k >= kListTasks;
+    if (listed) {
+        const std::int64_t pairs = static_cast<std::int64_t>(a.n_chunks) * k;
+        d.near.ensure(static_cast<std::size_t>(pairs), "near chunks");
+        d.near_flag.ensure(static_cast<std::size_t>(pairs), "near chunks");
+        d.near_count.ensure(static_cast<std::size_t>(k), "near chunks");
+        fill_i32_kernel<<<1, kBlock, 0, s>>>(d.near_count.get(), k, 0);
+        near_chunks_kernel<<<grid_for(pairs, kBlock / kWave), kBlock, 0, s>>>(a, d.near_flag.get(), d.near.get(),
+                                                                             d.near_count.get());
+        a.near_flag = d.near_flag.get();
+    }
     if (!d.parallel && !d.boxes) {
         node_given_kernel<<<capped((tasks + kBlock / kWave - 1) / (kBlock / kWave)), kBlock, pad, s>>>(a);
     } else if (k > 8 && a.n_chunks >= kWideMinChunks) {
@@ -1025,12 +1086,26 @@ void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int
         const auto go = [&](auto kernel, int groups) {
             kernel<<<capped((tasks + groups - 1) / groups), kDipoleThreads, pad, s>>>(a);
         };
-        if (tasks < kSplitTasks8)
-            d.parallel ? go(node_split_kernel<true, 8>, 1) : go(node_split_kernel<false, 8>, 1);
-        else if (tasks < kSplitTasks4)
-            d.parallel ? go(node_split_kernel<true, 4>, 2) : go(node_split_kernel<false, 4>, 2);
+        const auto split = [&](auto near) {
+            constexpr Near NEAR = decltype(near)::value;
+            if (tasks < kSplitTasks8)
+                go(node_split_kernel<NEAR, 8>, 1);
+            else if (tasks < kSplitTasks4)
+                go(node_split_kernel<NEAR, 4>, 2);
+            else
+                go(node_split_kernel<NEAR, 2>, 4);
+        };
+        if (d.parallel)
+            split(std::integral_constant<Near, Near::kPlain>{});
+        else if (listed)
+            split(std::integral_constant<Near, Near::kListed>{});
         else
-            d.parallel ? go(node_split_kernel<true, 2>, 4) : go(node_split_kernel<false, 2>, 4);
+            split(std::integral_constant<Near, Near::kSum>{});
+    }
+    if (listed) {
+        const std::int64_t blocks = (a.n_chunks + kBlock / kWave - 1) / (kBlock / kWave);
+        near_given_kernel<<<dim3(std::max(1u, max_blocks > 0 ? capped(blocks) / k : capped(blocks)), k), kBlock, pad, s>>>(
+            a, d.near.get(), d.near_count.get());
     }
     check(hipGetLastError(), "dA/dt launch");
 }

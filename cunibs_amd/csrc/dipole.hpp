@@ -46,6 +46,8 @@ struct DipoleSet {
     DeviceBuffer<float> dirs;      // (k, 3)
     DeviceBuffer<unsigned long long> far;  // (boxes, k) clusters taken through a box or its ancestors
     DeviceBuffer<float> values[kMaxBoxLevels];
+    DeviceBuffer<std::int32_t> near, near_count;  // (k, chunks) chunks summed in the caller's order; (k)
+    DeviceBuffer<unsigned char> near_flag;        // (chunks, k)
     PinnedStage stage_coil, stage_frames;
 };
 

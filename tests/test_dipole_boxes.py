@@ -84,6 +84,17 @@ def test_right_hand_sides_sum_to_zero(ctx, k):
     assert np.all(np.abs(b.sum(1)) <= 2.0 * 2.0**-24 * np.abs(b).max(1))
 
 
+@pytest.fixture(scope="module")
+def fine():
+    """A million nodes: deeper leaves, and the node pass that takes a block of workgroups per chunk."""
+    from cunibs_amd import fem
+    head = synthetic.shell_head(1.5, perturb_rms_mm=1.0, seed=2)
+    c = fem.SolverContext(head.nodes_mm, head.tet_nodes, head.tet_tags, head.skin_tris)
+    assert c.n_nodes >= 800000
+    yield c
+    c.free()
+
+
 def bent_coil(dipoles, tilt_deg=14.0):
     """Two wings tilted towards the head, whose moments differ in direction."""
     coil = synthetic.figure8_coil(seed=3, per_layer=-(-dipoles // 6))
@@ -93,6 +104,61 @@ def bent_coil(dipoles, tilt_deg=14.0):
         turn = np.array([[np.cos(t), 0.0, -np.sin(t)], [0.0, 1.0, 0.0], [np.sin(t), 0.0, np.cos(t)]])
         pos[wing], mom[wing] = pos[wing] @ turn.T, mom[wing] @ turn.T
     return pos, mom
+
+
+def rounding_bound(pos, mom, tf, nodes_mm):
+    """What FP32 may cost where a coil is summed as W x r - P with |r - s|^2 = |r|^2 + |s|^2 - 2 r.s, r and s
+    from the coil's origin: three roundings of |r|^2 + |s|^2 in a distance cubed, eight more of a term, and
+    one for each addition, of terms as large as w |m| (|r| + |s|)."""
+    s = pos @ tf[:3, :3].T
+    m = np.linalg.norm(mom, axis=1)
+    out = np.empty(nodes_mm.shape[0])
+    for i, x in enumerate(nodes_mm * 1e-3 - tf[:3, 3] * 1e-3):
+        d2 = ((x - s) ** 2).sum(1)
+        size = (x @ x) + (s * s).sum(1)
+        term = m * (np.sqrt(x @ x) + np.sqrt((s * s).sum(1))) / d2**1.5
+        out[i] = 0.1 * 2.0**-24 * (term * (3 * 1.5 * size / d2 + 8 + len(m))).sum()
+    return out
+
+
+@pytest.mark.parametrize("k,dipoles,bent", [(9, 2400, False), (17, 300, False), (32, 601, False), (9, 1801, True),
+                                            (17, 400, True), (32, 2400, True)])
+def test_wide_blocks_on_a_fine_mesh(fine, k, dipoles, bent):
+    """Against the closed form, and bit for bit against the same placements in narrow blocks, whose node
+    passes are others (and, for a bent coil, sum the near chunks themselves)."""
+    coil = synthetic.figure8_coil(seed=3, per_layer=-(-dipoles // 6))
+    pos, mom = bent_coil(dipoles) if bent else (coil.positions_m[:dipoles], coil.moments[:dipoles])
+    sites = synthetic.cap_sites(k, seed=k, distance_range_mm=(12.0, 14.0) if bent else (3.0, 8.0))
+    got, tf = nodal(fine, pos, mom, sites)
+    pick = np.random.default_rng(k).choice(fine.n_nodes, 400, replace=False)
+    for i in (0, k // 2, k - 1):
+        near = np.argsort(np.linalg.norm(fine.nodes_mm - tf[i][:3, 3], axis=1))[:200]
+        rows = np.concatenate([pick, near])
+        want = closed_form(pos, mom, tf[i], fine.nodes_mm[rows])
+        err = np.linalg.norm(got[i][rows] - want, axis=1)
+        if bent:
+            bound = rounding_bound(pos, mom, tf[i], fine.nodes_mm[rows])
+            assert np.all(err <= bound + 2e-5 * np.abs(want).max())
+        else:
+            assert np.linalg.norm(err) <= 6e-6 * np.linalg.norm(want)  # as above
+    for lo, hi in ((0, 1), (3, 5), (k - 8, k)):
+        part, _ = nodal(fine, pos, mom, sites[lo:hi])
+        np.testing.assert_array_equal(part, got[lo:hi])
+
+
+@pytest.mark.parametrize("k", [1, 12])
+def test_a_bent_coil_that_all_but_touches_nodes(ctx, k):
+    """Wings that reach into the scalp, within half a millimetre of nodes: the caller's order, whatever the
+    order of the dipoles does to their clusters."""
+    pos, mom = bent_coil(1500)
+    sites = synthetic.cap_sites(k, seed=7, distance_range_mm=(2.0, 3.0))
+    got, tf = nodal(ctx, pos, mom, sites)
+    i = k - 1
+    near = np.argsort(np.linalg.norm(ctx.nodes_mm - tf[i][:3, 3], axis=1))[:600]
+    want = closed_form(pos, mom, tf[i], ctx.nodes_mm[near])
+    err = np.linalg.norm(got[i][near] - want, axis=1)
+    print(f"k={k} n={ctx.n_nodes}: {np.linalg.norm(err) / np.linalg.norm(want):.2e} of the 2-norm")
+    assert np.all(err <= rounding_bound(pos, mom, tf[i], ctx.nodes_mm[near]))
 
 
 def test_a_general_coils_sweep_equals_its_blocks(ctx):
