@@ -44,16 +44,31 @@ constexpr double kUpperDistance = 3.5;  // admissible distance over the largest 
 constexpr double kLeafDistance = 5.5;
 constexpr double kCloseMm = 10.0;
 
-// The box method is taken from these sizes up. Below them most clusters are near every box that
-// holds enough nodes to pay, and the launches of the levels cost more than the pairs they save.
+// The box method is taken from these sizes up; below them the launches of the levels, and boxes that are
+// near most clusters, cost more than the pairs they save. Whether it pays depends on the block's width
+// too, but a placement's sum must not, so the lines lie where the widths from 1 to 32 balance, later where
+// the leaves are one level deeper. Flat coil, us without and with boxes at widths 1, 4, 16 and 32: 400
+// dipoles at 125,000 nodes 34 87 284 530 and 57 114 302 547, at 213,000 46 136 454 879 and 66 138 402 732;
+// 600 at 125,000 43 117 400 772 and 67 137 377 677; 400 at 412,000 69 236 854 1684 and 117 283 845 1922,
+// 600 there 96 343 1255 2471 and 129 319 964 2129; 260 at 966,000 107 380 1251 2489 and 125 385 1026 2194.
+// Moments that differ (near chunks take every dipole either way): 600 dipoles at 213,000 nodes 76 205 701
+// 1367 and 122 249 739 1278; 1,800 at 125,000 165 370 1239 2413 and 265 470 1338 2239; 964 at 412,000 182
+// 636 2218 4275 and 283 598 1807 3652; 400 at 667,000 114 382 1412 2787 and 184 460 1407 2790; 260 at
+// 966,000 105 366 1337 2644 and 161 469 1432 2866.
 constexpr std::int64_t kBoxMinNodes = 100000;
 constexpr std::int64_t kBoxMinDipoles = 256;
-// Leaves one level deeper from here: 60 to 500 nodes a leaf box against its 216 points.
+constexpr std::int64_t kBoxMinPairs = 80000000, kBoxMinPairsDeep = 200000000;
+constexpr std::int64_t kBoxMinGeneralPairs = 240000000, kBoxMinGeneralPairsDeep = 320000000;
+// Leaves one level deeper from here. Sweeps 16 wide at 412,000 nodes, 4,000 dipoles: 28.1 ms with the
+// shallower leaves and 27.6 deeper (flat coil), 34.2 and 32.0 (moments that differ), 400 dipoles 23.5 and
+// 24.1; at 214,000 nodes, 8,700 chunks deeper against 4,500, most leaves would hold fewer nodes than the
+// 216 points they take. At the deepest level a placement's box values take up to 100 MB.
 constexpr std::int64_t kBoxDeepNodes = 400000;
 constexpr std::int64_t kBoxDeeperNodes = 3200000;
 
-// Chunks from which a wide block's node pass takes a block per chunk (at 412,000 nodes, 6,600 chunks: 16
-// and 32 placements of 1,800 dipoles 1357 and 2655 us so, 1333 and 2508 with waves sharing a chunk), and
+// Chunks from which a wide block's node pass takes a block per chunk (4,500 chunks at 213,000 nodes: 16
+// and 32 placements of 1,800 dipoles 1102 and 2116 us so, 994 and 1836 with waves sharing a chunk; 8,000
+// at 412,000: 1623 and 3323 so, 1659 and 3432 shared), and
 // (chunk, placement) tasks below which eight and four waves share one (one placement at 7,400 nodes has
 // 116 tasks: 15 us for 964 dipoles).
 constexpr int kWideMinChunks = 8192;
@@ -73,10 +88,10 @@ static_assert(kListTasks <= 9 * kWideMinChunks, "node_wide_kernel leaves near ch
 // 966,000 nodes 97.3 and 96.4; a general coil's at 95,000 nodes 28.3 and 25.2). The box and node passes
 // of many dipoles whose moments differ take longer than the solves beside them, and then take more of
 // the machine (32-wide sweeps at 138,000 nodes: 4,000 dipoles 32.3 ms with the wide pad, 28.4 so, 2,600
-// 26.3 and 24.9, 1,800 22.6 and 22.8).
+// 26.3 and 24.9, 1,800 22.6 and 22.8; of 4,000, 8 wide 13.5 and 12.8, 4 wide 9.6 and 10.0).
 constexpr std::size_t kBesideLds = 60 * 1024;
 constexpr std::size_t kBesideHeavyLds = 24 * 1024;
-constexpr int kHeavyDipoles = 2304;
+constexpr int kHeavyDipoles = 2304, kHeavyWidth = 8;
 
 // tables layout (floats): points of order 8, points of order 6, then for child order 8 and 6 the
 // matrices T[half][child point][parent point] (parent order 8).
@@ -846,6 +861,7 @@ void split_clusters(Site* p, Site* tmp, int n_dip, int q0, int q1) {
 
 void build_box_tree(BoxTree& t, const double* nodes_mm, std::int64_t n, hipStream_t s) {
     t.levels = 0;
+    t.n = n;
     if (n < kBoxMinNodes) return;
     const int leaf_level = n >= kBoxDeeperNodes ? 5 : n >= kBoxDeepNodes ? 4 : 3;
     const int levels = leaf_level - kTopLevel + 1;
@@ -934,7 +950,10 @@ void set_coil(DipoleSet& d, const BoxTree& t, const double* pos_m, const double*
     require(n_dip >= 1 && n_dip < (1ll << 31) / kClusters, "dipole count out of range");
     d.n = static_cast<int>(n_dip);
     d.parallel = common_moment_direction(mom, n_dip, d.dir);
-    d.boxes = t.levels > 0 && n_dip >= kBoxMinDipoles;
+    const bool deep = t.n >= kBoxDeepNodes;
+    const std::int64_t pairs = d.parallel ? (deep ? kBoxMinPairsDeep : kBoxMinPairs)
+                                          : (deep ? kBoxMinGeneralPairsDeep : kBoxMinGeneralPairs);
+    d.boxes = t.levels > 0 && n_dip >= kBoxMinDipoles && t.n * n_dip >= pairs;
     std::vector<std::int32_t> order(static_cast<std::size_t>(n_dip));
     for (int i = 0; i < d.n; ++i) order[i] = i;
     if (d.boxes) {
@@ -989,7 +1008,8 @@ void set_coil(DipoleSet& d, const BoxTree& t, const double* pos_m, const double*
 void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int64_t n, const double* tf, int k, int K,
                 float scale, float* out, int max_blocks, bool beside, hipStream_t s) {
     if (n <= 0 || k <= 0) return;
-    const std::size_t pad = !beside ? 0 : d.boxes && !d.parallel && d.n >= kHeavyDipoles ? kBesideHeavyLds : kBesideLds;
+    const bool heavy = d.boxes && !d.parallel && d.n >= kHeavyDipoles && k >= kHeavyWidth;
+    const std::size_t pad = !beside ? 0 : heavy ? kBesideHeavyLds : kBesideLds;
     require(d.n >= 1, "no coil has been set");
     d.frames.ensure(16 * static_cast<std::size_t>(k), "coil frames");
     d.origin.ensure(3 * static_cast<std::size_t>(k), "coil origins");

@@ -14,6 +14,7 @@ constexpr int kLeafOrder = 6;       // ... and of the leaf boxes
 // contiguous run), from kTopLevel to the leaf level; levels = 0 where the mesh is too small for them.
 struct BoxTree {
     int levels = 0;
+    std::int64_t n = 0;  // nodes
     int n_box[kMaxBoxLevels] = {};
     int first[kMaxBoxLevels] = {};       // position of a level's boxes in the arrays below
     int total = 0;

@@ -90,7 +90,7 @@ def fine():
     from cunibs_amd import fem
     head = synthetic.shell_head(1.5, perturb_rms_mm=1.0, seed=2)
     c = fem.SolverContext(head.nodes_mm, head.tet_nodes, head.tet_tags, head.skin_tris)
-    assert c.n_nodes >= 800000
+    assert c.n_nodes >= 800000  # more than 8,192 chunks of 64 nodes
     yield c
     c.free()
 
@@ -175,3 +175,60 @@ def test_a_general_coils_sweep_equals_its_blocks(ctx):
             np.testing.assert_array_equal(sweep["metrics"], np.stack(blocks))
     finally:
         ctx.set_tuning(coil_blocks=0)
+
+
+@pytest.mark.parametrize("bent,pairs,pairs_deep", [(False, 80000000, 200000000), (True, 240000000, 320000000)])
+def test_both_sides_of_the_box_rule(ctx, bent, pairs, pairs_deep):
+    """The last coil without boxes and the first with them, against the closed form."""
+    first = max(256, -(-(pairs_deep if ctx.n_nodes >= 400000 else pairs) // ctx.n_nodes))
+    for dipoles in (first - 1, first) if first < 4000 else (2000,):
+        coil = synthetic.figure8_coil(seed=3, per_layer=-(-dipoles // 6))
+        pos, mom = coil.positions_m[:dipoles].copy(), coil.moments[:dipoles].copy()
+        if bent:
+            mom += 0.1 * np.abs(mom).max() * np.random.default_rng(1).standard_normal(mom.shape)
+        got, tf = nodal(ctx, pos, mom, synthetic.cap_sites(2, seed=3))
+        pick = np.random.default_rng(2).choice(ctx.n_nodes, 400, replace=False)
+        want = closed_form(pos, mom, tf[1], ctx.nodes_mm[pick])
+        err = np.linalg.norm(got[1][pick] - want, axis=1)
+        assert np.linalg.norm(err) <= 6e-6 * np.linalg.norm(want)  # as above
+        assert err.max() <= 2e-5 * np.abs(want).max()
+
+
+def box_mesh(cells):
+    """A box of 1 mm cells, six positively oriented tetrahedra each, and two triangles of its top."""
+    side = cells + 1
+    axis = np.arange(side, dtype=np.float64)
+    nodes = np.stack(np.meshgrid(axis, axis, axis, indexing="ij"), -1).reshape(-1, 3)
+    i = np.arange(cells, dtype=np.int32)
+    base = ((i[:, None, None] * side + i[None, :, None]) * side + i).reshape(-1)
+    step = np.array([side * side, side, 1], np.int32)
+    tets = np.empty((6, base.size, 4), np.int32)
+    for q, (a, b, odd) in enumerate(((0, 1, 0), (0, 2, 1), (1, 0, 1), (1, 2, 0), (2, 0, 0), (2, 1, 1))):
+        path = [base, base + step[a], base + step[a] + step[b], base + step.sum()]
+        if odd:
+            path[1], path[2] = path[2], path[1]
+        tets[q] = np.stack(path, 1)
+    top = cells
+    corner = [(x * side + y) * side + top for x, y in ((0, 0), (cells, 0), (cells, cells), (0, cells))]
+    return nodes, tets.reshape(-1, 4), np.array([[corner[0], corner[1], corner[2]], [corner[0], corner[2], corner[3]]],
+                                               np.int32)
+
+
+def test_the_deepest_boxes():
+    from cunibs_amd import fem
+    nodes, tets, skin = box_mesh(147)
+    assert nodes.shape[0] >= 3200000
+    c = fem.SolverContext(nodes, tets, np.full(tets.shape[0], 2, np.int32), skin)
+    try:
+        coil = synthetic.figure8_coil(seed=3, per_layer=400)
+        at = np.array([73.0, 73.0, 147.0])
+        sites = [(at + [10.0 * i, 0.0, 0.0], at + [10.0 * i, 50.0, 0.0], 4.0) for i in range(9)]
+        for k in (1, 9):
+            got, tf = nodal(c, coil.positions_m, coil.moments, sites[:k])
+            pick = np.random.default_rng(k).choice(c.n_nodes, 400, replace=False)
+            want = closed_form(coil.positions_m, coil.moments, tf[k - 1], c.nodes_mm[pick])
+            err = np.linalg.norm(got[k - 1][pick] - want, axis=1)
+            assert np.linalg.norm(err) <= 6e-6 * np.linalg.norm(want)  # as above
+            assert err.max() <= 2e-5 * np.abs(want).max()
+    finally:
+        c.free()
