@@ -33,15 +33,10 @@ class OutputCopy {
 
     // dst (host) = src (device), `bytes` long, after the work queued on `s`; complete on return.
     void run(void* dst, const void* src, std::size_t bytes, hipStream_t s) {
-        if (bytes < kMinBytes) {
+        if (bytes < kMinBytes || !pinned()) {
             if (bytes) check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s), "output copy");
             sync(s, "output copy");
             return;
-        }
-        if (!ring_) {
-            void* p = nullptr;
-            check(hipHostMalloc(&p, kChunk * kSlots), "output ring");
-            ring_ = static_cast<char*>(p);
         }
         for (auto& e : ev_)
             if (!e) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "output event");
@@ -65,6 +60,13 @@ class OutputCopy {
     }
 
   private:
+    // The ring, allocated at its first use; where there is no pinned memory to be had the copy is plain.
+    bool pinned() {
+        void* p = nullptr;
+        if (!ring_ && hipHostMalloc(&p, kChunk * kSlots) == hipSuccess) ring_ = static_cast<char*>(p);
+        if (!ring_) (void)hipGetLastError();
+        return ring_ != nullptr;
+    }
     // 1 MB chunks take the link 20 us and a worker up to 0.2 ms with their page faults.
     static constexpr std::size_t kChunk = std::size_t{1} << 20;
     static constexpr std::size_t kSlots = 12;

@@ -1,14 +1,34 @@
 """Fields copied through the ring of pinned chunks (csrc/output_copy.hpp) against those below its
-smallest size: the norm of E, element by element, is the |E| of the same block."""
+smallest size: the norm of E, element by element, is the |E| of the same block. The hand-over itself, with
+every byte looked at, on the CPU."""
 
 from __future__ import annotations
+
+import subprocess
+from pathlib import Path
 
 import numpy as np
 import pytest
 
 from cunibs_amd import synthetic
 
-pytestmark = pytest.mark.gpu
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def host_program(tmp_path_factory):
+    out = tmp_path_factory.mktemp("copy") / "output_copy_host"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'cunibs_amd' / 'csrc'}", str(ROOT / "tests" / "output_copy_host.cpp"), "-o", str(out)],
+                   check=True, capture_output=True, text=True)
+    return out
+
+
+@pytest.mark.parametrize("failing,no_pinned", [(-1, 0), (-1, 1)])
+def test_ring_hands_over_every_byte(host_program, failing, no_pinned):
+    """Whole, and without pinned memory."""
+    done = subprocess.run([str(host_program), str(failing), str(no_pinned)], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout + done.stderr
 
 
 @pytest.fixture(scope="module")
@@ -20,6 +40,7 @@ def ctx():
     c.free()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("k", [1, 2, 4, 5])  # E of 3.7, 7.4, 14.9 and 18.6 MB: below the ring, within it, past it
 def test_fields_through_the_ring(ctx, k):
     from cunibs_amd import fem
