@@ -12,7 +12,6 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -84,8 +83,9 @@ class OutputCopy {
             workers_.reserve(static_cast<std::size_t>(want));
             try {
                 for (int w = 0; w < want; ++w) workers_.emplace_back([this] { work(); });
-            } catch (const std::system_error&) {
-                // Fewer threads, or none: finish() and emptied() then copy on this one.
+            } catch (...) {
+                // No thread or no memory for one: with fewer, or none, finish() and emptied() copy on this
+                // one. (Left to itself the exception would meet threads that are running.)
             }
         }
         ~Ring() {

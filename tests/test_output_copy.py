@@ -24,9 +24,10 @@ def host_program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("failing,no_pinned", [(-1, 0), (-1, 1)])
+@pytest.mark.parametrize("failing,no_pinned", [(-1, 0), (-1, 1), (2, 0), (3, 0), (5, 0), (7, 0)])
 def test_ring_hands_over_every_byte(host_program, failing, no_pinned):
-    """Whole, and without pinned memory."""
+    """Whole, without pinned memory, and when an allocation of one of the threads fails (the first two are
+    the copy's own tables)."""
     done = subprocess.run([str(host_program), str(failing), str(no_pinned)], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stdout + done.stderr
 
