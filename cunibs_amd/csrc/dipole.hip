@@ -947,7 +947,7 @@ void build_box_tree(BoxTree& t, const double* nodes_mm, std::int64_t n, hipStrea
 
 void set_coil(DipoleSet& d, const BoxTree& t, const double* pos_m, const double* mom,
               std::int64_t n_dip, hipStream_t s) {
-    require(n_dip >= 1 && n_dip < (1ll << 31) / kClusters, "dipole count out of range");
+    require(n_dip >= 1 && n_dip <= INT32_MAX / 6, "dipole count out of range");
     d.n = static_cast<int>(n_dip);
     d.parallel = common_moment_direction(mom, n_dip, d.dir);
     const bool deep = t.n >= kBoxDeepNodes;

@@ -194,6 +194,25 @@ def test_both_sides_of_the_box_rule(ctx, bent, pairs, pairs_deep):
         assert err.max() <= 2e-5 * np.abs(want).max()
 
 
+def test_a_coil_of_more_than_two_to_the_25_dipoles():
+    """Nearly all of them without a moment."""
+    from cunibs_amd import fem
+    head = synthetic.shell_head(10.0, seed=2)
+    n = 2**25 + 1
+    rng = np.random.default_rng(0)
+    live = np.append(rng.choice(n - 1, 63, replace=False), n - 1)
+    pos, mom = np.zeros((n, 3)), np.zeros((n, 3))
+    pos[live], mom[live, 2] = rng.uniform(-0.03, 0.03, (64, 3)) * [1.0, 1.0, 0.1], 1e-3
+    ctx = fem.SolverContext(head.nodes_mm, head.tet_nodes, head.tet_tags, head.skin_tris)
+    try:
+        got, tf = nodal(ctx, pos, mom, synthetic.cap_sites(1, seed=1, distance_mm=8.0))
+        want = closed_form(pos[live], mom[live], tf[0], ctx.nodes_mm)
+    finally:
+        ctx.free()
+    err = np.linalg.norm(got[0] - want, axis=1)
+    assert np.linalg.norm(err) <= 6e-6 * np.linalg.norm(want)  # as above: a zero term adds no rounding
+
+
 def box_mesh(cells):
     """A box of 1 mm cells, six positively oriented tetrahedra each, and two triangles of its top."""
     side = cells + 1
