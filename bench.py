@@ -627,9 +627,7 @@ def main() -> int:
         f"({achieved:.0f} GB/s), V-cycle {vc_ms * 1e3:.1f} us ({vc_achieved:.0f} GB/s), "
         f"iteration {it_ms * 1e3:.1f} us")
     n_dip = pos.shape[0]
-    dadt_flop = 20.0 * ctx.n_nodes * n_dip
     dadt_ms = dadt_phase_ms
-    dadt_tf = dadt_flop / (dadt_ms * 1e-3) / 1e12 if dadt_ms > 0 else float("nan")
     dadt_iso = round(ctx.bench_dadt(pos, mom, sites[0], k=8, reps=3) / 8, 4)
     isolated = None
     if args.isolated:
@@ -722,15 +720,11 @@ def main() -> int:
             "algorithmic_bytes": vc_bytes,
             "degree": degree,
         },
-        "dadt_roofline": {
-            "bound": "valu",
-            "achieved": round(dadt_tf, 2),
-            "peak": 157.3,
-            "unit": "TFLOP/s",
-            "frac": round(dadt_tf / 157.3, 4),
+        # No rate: the box method sums a part of the n x D pairs, which part depends on where the coil is.
+        "dadt": {
             "avg_ms_per_placement": round(dadt_ms, 4),
-            "flop_per_placement": dadt_flop,
             "isolated_ms_per_placement": dadt_iso,
+            "direct_pairs_per_placement": ctx.n_nodes * n_dip,
         },
         "iteration_us": round(it_ms * 1e3, 2),
         "isolated_us": isolated,
