@@ -116,6 +116,30 @@ def test_asking_for_the_potential_changes_nothing_else(head8, coil):
 
 
 @pytest.mark.gpu
+def test_the_spread_of_few_draws_matches_fp64_solves(head8, coil, oracle_mod):
+    """Ten draws' standard deviation, element by element. A solve to 1e-6 leaves 2e-5 of a draw's field at
+    most, and a standard deviation moves by no more than that of the draws' errors, which is sqrt(n / (n - 1))
+    of their root mean square."""
+    from cunibs_amd import fem, synthetic, uq
+    mesh = (head8.nodes_mm, head8.tet_nodes, head8.tet_tags, head8.skin_tris)
+    site = synthetic.SPHERE_SITE
+    ctx = fem.SolverContext(*mesh)
+    try:
+        tags = ctx.uq_prepare(coil.positions_m, coil.moments, site, 1e6)
+        sigma = uq.draw_lognormal(tags, 10, 0.2, seed=13)
+        ctx.uq_solve(sigma, magnitude=False)
+        mean, var, _ = ctx.uq_moments()
+    finally:
+        ctx.free()
+    want = np.stack([oracle_mod.solve_site(
+        oracle_mod.build_context(*mesh, conductivity={**fem.TISSUE_CONDUCTIVITY, **dict(zip(tags, map(float, row)))}),
+        coil.positions_m, coil.moments, site, 1e6, tol=1e-12)["magnE"] for row in sigma])
+    spread = want.std(axis=0, ddof=1)
+    assert np.linalg.norm(mean - want.mean(axis=0)) <= 2e-5 * np.linalg.norm(want.mean(axis=0))
+    assert np.linalg.norm(np.sqrt(var) - spread) <= 2e-5 * np.sqrt(10.0 / 9.0) * np.linalg.norm(mean)
+
+
+@pytest.mark.gpu
 def test_draws_carry_no_net_current(head8, coil):
     """A draw's right-hand side is brought to a zero sum after its tissues' vectors are combined, so its
     potential is off by no more of a constant than a block's of the same conductivities (1e-6 of its norm
