@@ -428,18 +428,30 @@ __device__ __forceinline__ Chunk chunk_at(const NodeArgs& a, int chunk) {
     return {n0, static_cast<int>(min(static_cast<std::int64_t>(kWave), a.n - n0)), -1, chunk};
 }
 
-// Whether some cluster (lane q testing cluster q) of placement c lies within kCloseMm of this chunk.
-__device__ __forceinline__ bool close_by(const NodeArgs& a, const Chunk& ch, int c) {
+// The middle of cluster q of placement c (m).
+__device__ __forceinline__ void cluster_at(const NodeArgs& a, int c, int q, double* p) {
     const double* f = a.frames + 16 * c;
-    const double* sp = a.spheres + 4 * (threadIdx.x & (kWave - 1));
-    const double* ball = a.ball + 4 * static_cast<std::int64_t>(ch.id);
+    const double* sp = a.spheres + 4 * q;
+    for (int r = 0; r < 3; ++r)
+        p[r] = (sp[0] * f[4 * r] + sp[1] * f[4 * r + 1] + sp[2] * f[4 * r + 2]) + f[4 * r + 3] * 1e-3;
+}
+
+// Whether a cluster around p (m) lies within kCloseMm of a chunk's ball (mm).
+__device__ __forceinline__ bool within_close(const double* ball, const double* p, double radius) {
     double d2 = 0.0;
     for (int r = 0; r < 3; ++r) {
-        const double p = (sp[0] * f[4 * r] + sp[1] * f[4 * r + 1] + sp[2] * f[4 * r + 2]) + f[4 * r + 3] * 1e-3;
-        const double d = ball[r] * 1e-3 - p;
+        const double d = ball[r] * 1e-3 - p[r];
         d2 += d * d;
     }
-    return __ballot(sqrt(d2) - sp[3] < (kCloseMm + ball[3]) * 1e-3) != 0;
+    return sqrt(d2) - radius < (kCloseMm + ball[3]) * 1e-3;
+}
+
+// Whether some cluster (lane q testing cluster q) of placement c lies within kCloseMm of this chunk.
+__device__ __forceinline__ bool close_by(const NodeArgs& a, const Chunk& ch, int c) {
+    const int q = threadIdx.x & (kWave - 1);
+    double p[3];
+    cluster_at(a, c, q, p);
+    return __ballot(within_close(a.ball + 4 * static_cast<std::int64_t>(ch.id), p, a.spheres[4 * q + 3])) != 0;
 }
 
 // How a node pass treats the chunks near a coil: a planar coil's like any other; else it sums every dipole
@@ -759,18 +771,33 @@ __global__ void __launch_bounds__(kBlock) node_given_kernel(NodeArgs a) {
     }
 }
 
-// flag[chunk, c]: whether placement c takes the chunk in the caller's order; near[c] = those chunks, in no
-// order. One wavefront per (chunk, placement). `count` starts at zero.
+// flag[chunk, c]: whether placement c = blockIdx.y takes the chunk in the caller's order (close_by, one
+// chunk a lane); near[c] = those chunks, in no order. `count` starts at zero; one addition a wavefront
+// (one a near chunk took 200 us of 16 placements at 966,000 nodes).
 __global__ void __launch_bounds__(kBlock) near_chunks_kernel(NodeArgs a, unsigned char* __restrict__ flag,
                                                              std::int32_t* __restrict__ near,
                                                              std::int32_t* __restrict__ count) {
-    const std::int64_t w = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
-    if (w >= static_cast<std::int64_t>(a.n_chunks) * a.k) return;  // whole wavefronts
-    const int chunk = static_cast<int>(w / a.k), c = static_cast<int>(w % a.k);
-    const bool given = close_by(a, chunk_at(a, chunk), c);
-    if ((threadIdx.x & (kWave - 1)) != 0) return;
-    flag[w] = given;
-    if (given) near[static_cast<std::int64_t>(c) * a.n_chunks + atomicAdd(count + c, 1)] = chunk;
+    __shared__ double sphere[kClusters][4];
+    const int c = blockIdx.y, t = threadIdx.x;
+    if (t < kClusters) {
+        cluster_at(a, c, t, sphere[t]);
+        sphere[t][3] = a.spheres[4 * t + 3];
+    }
+    __syncthreads();
+    const int chunk = static_cast<int>(blockIdx.x) * kBlock + t;
+    bool given = false;
+    if (chunk < a.n_chunks) {
+        const double* ball = a.ball + 4 * static_cast<std::int64_t>(chunk);
+        const double b[4] = {ball[0], ball[1], ball[2], ball[3]};
+        for (int q = 0; q < kClusters && !given; ++q) given = within_close(b, sphere[q], sphere[q][3]);
+        flag[static_cast<std::int64_t>(chunk) * a.k + c] = given;
+    }
+    const unsigned long long m = __ballot(given);
+    if (m == 0) return;  // whole wavefronts
+    const int lane = t & (kWave - 1);
+    int at = lane == 0 ? atomicAdd(count + c, __popcll(m)) : 0;
+    at = __shfl(at, 0, kWave) + __popcll(m & ((1ull << lane) - 1ull));
+    if (given) near[static_cast<std::int64_t>(c) * a.n_chunks + at] = chunk;
 }
 
 // Placement blockIdx.y at its near chunks, one a wavefront: in the node passes of a wide block the waves
@@ -1089,8 +1116,8 @@ void dadt_block(DipoleSet& d, const BoxTree& t, const double* nodes_mm, std::int
         d.near_flag.ensure(static_cast<std::size_t>(pairs), "near chunks");
         d.near_count.ensure(static_cast<std::size_t>(k), "near chunks");
         fill_i32_kernel<<<1, kBlock, 0, s>>>(d.near_count.get(), k, 0);
-        near_chunks_kernel<<<grid_for(pairs, kBlock / kWave), kBlock, 0, s>>>(a, d.near_flag.get(), d.near.get(),
-                                                                             d.near_count.get());
+        near_chunks_kernel<<<dim3(grid_for(a.n_chunks), static_cast<unsigned>(k)), kBlock, 0, s>>>(
+            a, d.near_flag.get(), d.near.get(), d.near_count.get());
         a.near_flag = d.near_flag.get();
     }
     if (!d.parallel && !d.boxes) {
