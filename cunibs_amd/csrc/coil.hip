@@ -350,48 +350,45 @@ __global__ void combined_sums_kernel(const float* __restrict__ B, std::int64_t n
 // The right-hand side of a field without sources sums to zero over all nodes; its FP32 rounding
 // does not, and whatever is left (5e-8 of the norm) flows to the ground node, which shifts the whole
 // potential by 1e-6 to 4e-5 of its norm. The sum of each column is taken back from kBalanceRows rows
-// spread over the mesh, a thread rounding each, and what their roundings leave from the first of them,
-// which leaves one rounding of its entry (the potential's error: 3e-7, that of the solve). One block per
-// column; the sum does not depend on the block's width. With one thread walking the rows and one load of
-// the sums in flight it took 8 us for a column at 7,400 nodes and 22 at 1.0M, now 4 and 8.
+// spread over the mesh, each rounded value's error carried to the next, which leaves less than one
+// rounding of one entry (the potential's error: 3e-7, that of the solve). One block per column; the
+// sum does not depend on the block's width. The carried chain takes 4 us whatever the mesh; the rows
+// rounded side by side, with the remainder in one of them, took none of that, but any other rounding
+// moves single potentials by the solve's error (2e-6 at five placements of 127,000 nodes).
 constexpr int kBalanceRows = kBlock;
 
 __global__ void __launch_bounds__(kBlock) balance_rhs_kernel(const double* __restrict__ sums, std::int64_t blocks,
                                                              std::int64_t n, int K, int ground, float* __restrict__ B,
                                                              float* __restrict__ b_full) {
     __shared__ double s[kBlock];
+    __shared__ float v[kBalanceRows];
     const int c = blockIdx.x, t = threadIdx.x;
-    const auto total = [&](double v) {  // of every thread's v, a fixed tree
-        s[t] = v;
-        __syncthreads();
-        for (int w = kBlock / 2; w > 0; w >>= 1) {
-            if (t < w) s[t] += s[t + w];
-            __syncthreads();
-        }
-        const double out = s[0];
-        __syncthreads();
-        return out;
-    };
     double acc = 0.0;
 #pragma unroll 8
     for (std::int64_t b = t; b < blocks; b += kBlock) acc += sums[b * K + c];  // eight loads in flight
-    const double net = total(acc);
-    if (net == 0.0) return;
+    s[t] = acc;
     const std::int64_t nr = n - 1;
     const int rows = static_cast<int>(min(static_cast<std::int64_t>(kBalanceRows), nr));
     const std::int64_t row = static_cast<std::int64_t>(t) * nr / rows;
-    double left = 0.0;
-    float v = 0.f;
-    if (t < rows) {
-        const double x = static_cast<double>(B[row * K + c]) - net / rows;
-        v = static_cast<float>(x);
-        left = x - static_cast<double>(v);
+    if (t < rows) v[t] = B[row * K + c];
+    __syncthreads();
+    for (int w = kBlock / 2; w > 0; w >>= 1) {
+        if (t < w) s[t] += s[t + w];
+        __syncthreads();
     }
-    left = total(left);
-    if (t == 0) v = static_cast<float>(static_cast<double>(v) + left);
+    if (t == 0 && s[0] != 0.0) {
+        const double share = -s[0] / rows;
+        double carry = 0.0;
+        for (int i = 0; i < rows; ++i) {
+            const double x = static_cast<double>(v[i]) + (share + carry);
+            v[i] = static_cast<float>(x);
+            carry = x - static_cast<double>(v[i]);
+        }
+    }
+    __syncthreads();
     if (t < rows) {
-        B[row * K + c] = v;
-        if (b_full != nullptr) b_full[c * n + row + (row >= ground)] = v;
+        B[row * K + c] = v[t];
+        if (b_full != nullptr) b_full[c * n + row + (row >= ground)] = v[t];
     }
 }
 
