@@ -19,7 +19,9 @@
 // A coil whose moments differ in direction may be bent around the head until its dipoles all but
 // touch nodes. There W x r - P (below) cancels to the last digits, so the runs of 64 nodes within
 // kCloseMm of such a coil's clusters, and every node of a mesh without boxes, take all its dipoles in
-// the caller's order, one sum per node.
+// the caller's order, one sum per node. Half a millimetre from a dipole that sum itself is off by up to
+// 1e-3 of the 2-norm over the nearest 600 nodes (4e-6 to 1e-4 on finer meshes); any other order or form
+// gives other last digits, 2.5 % of E in places.
 //
 // The sum of a placement does not depend on the block it is in: the dipoles are always summed in
 // the same 8 slices, each in order, and the slices added in order, whichever waves take them.
